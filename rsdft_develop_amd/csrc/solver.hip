@@ -111,13 +111,25 @@ __global__ __launch_bounds__(kThreads) void k_multidot(DotArgs<W> a, int64_t N, 
   }
 }
 
+// out[t] = alpha * sum_s partial[t nseg + s].  Eight lanes per sum: one
+// thread per sum walks nseg dependent loads (5.6 us for 20 sums of 64, a
+// fifth of a small cell's CG call); a fixed order either way.
+constexpr int kRedLanes = 8;
 __global__ void k_reduce_partials(const double *__restrict__ partial, int nseg, int count,
                                   double alpha, double *__restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= count) return;
+  const int t = (blockIdx.x * blockDim.x + threadIdx.x) / kRedLanes, l = threadIdx.x % kRedLanes;
   double v = 0.0;
-  for (int s = 0; s < nseg; ++s) v += partial[int64_t(t) * nseg + s];
-  out[t] = alpha * v;
+  if (t < count)
+    for (int s = l; s < nseg; s += kRedLanes) v += partial[int64_t(t) * nseg + s];
+#pragma unroll
+  for (int o = kRedLanes / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, kRedLanes);
+  if (t < count && l == 0) out[t] = alpha * v;
+}
+
+void reduce_partials(rsg_ctx *ctx, const double *partial, int nseg, int count, double alpha, double *out) {
+  constexpr int per = 256 / kRedLanes;
+  hipLaunchKernelGGL(k_reduce_partials, dim3((count + per - 1) / per), dim3(256), 0, ctx->stream, partial, nseg, count,
+                     alpha, out);
 }
 
 // --------------------------------------------------------- band-wise updates
@@ -815,6 +827,288 @@ __global__ __launch_bounds__(kThreads) void k_pczv(PzArgs<W, S> A, PzGeom q, W c
   block_partial(acc, A.partial, b, zr * q.nq + qb, q.nseg);
 }
 
+// ---- hprsdft preconditioner of up to three steps, recomputing passes ----
+// The CG iteration on A = -1/2 lap_7 from x0 = g in terms of its directions:
+//   p_0 = r_0 = g - A g,
+//   r_k = p_{k-1} - b_{k-2} p_{k-2} - a_{k-1} A p_{k-1},  p_k = r_k + b_{k-1} p_{k-1},
+//   x   = g + sum_k a_k p_k.
+// A pass forms p_k from the stored p_{k-1} (and p_{k-2}) on its tile and a
+// one-point rim around it, and applies A to it in the same sweep, so that
+// the products of p_k with A p_k come without reading p_k back; the last
+// direction is formed twice and never stored.  Per call with three steps 10
+// vector streams (g -> p_0 2, p_0 -> p_1 2, p_1 p_0 -> products of p_2 2,
+// g p_0 p_1 -> x 4) against 24 for one sweep per CG update (k_pczv).
+// <r_{k+1}, r_{k+1}> comes from <r_k, r_k> - 2 a <r_k, A p_k> + a^2 <A p_k,
+// A p_k>, all sums of the pass; where it falls below kPsGuard of <r_k, r_k>
+// (the difference would lose more than two digits) the band's blocks sum it
+// directly in a sweep of their own (kPsRho); the other bands' blocks of that
+// sweep only finish the scalars and leave.
+//
+// A block owns all of x for ty rows of one band and a run of z-planes; each
+// thread holds VP adjacent points of one row (rows past the tile's edge are
+// the rim) and walks z with the planes z-1, z, z+1 of the input and of p_k
+// in registers.  In-plane neighbours come through LDS (double-buffered, one
+// barrier per plane).  Bound: memory traffic; ty rows read ty + 4 (ty + 2).
+// Si216 (1.26M points, 480 bands, FP64): four calls of an eigensolver pass
+// take 63 ms less than as 24 streams (103 ms); Si64 FP32 CG call and
+// Gram-Schmidt 15.0 -> 11.4 ms, 75 x 38 x 70 with 77 bands (one point per
+// thread) 11.2 -> 8.8 ms per pass, 36^3 with 20 bands 1.16 -> 0.94 ms.
+enum PsOp { kPsFirst, kPsNext1, kPsNext2, kPsRho1, kPsRho2, kPsFin2, kPsFin3 };
+constexpr double kPsGuard = 1e-2;
+constexpr int kPsScal = 16;  // per band: a[0..2], b[3..4], <r_k, r_k> [5..7], direct-sum flag [8]
+
+template <typename W> struct PsArgs {
+  const W *s1, *s2, *g;  // stencil input, the direction before it, g (x passes)
+  W *out;                // p_k (null: not stored), or x
+  int64_t ld1, ldo;      // leading dimensions of s1 and out
+  const double *part_in, *part_rho;  // sums of the pass before, and of its direct <r, r> sweep
+  double *part, *scal;
+  int nin, nrho, k;      // segments of part_in and part_rho; index of the direction the pass is about
+  int *above;            // set when some <r_0, r_0> is not below the early-exit bound
+};
+
+struct PsGeom {
+  int n1, n2, n3, ty, nty, zlen, nzr;
+  int64_t N, n12, ld;
+};
+
+__device__ inline double ps_sum(const double *__restrict__ part, int b, int nseg, int nd, int d) {
+  double v = 0.0;
+  for (int s = int(threadIdx.x & 63); s < nseg; s += 64) v += part[(int64_t(b) * nseg + s) * nd + d];
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+__device__ inline double ps_alpha(double rr, double pap) { return pap != 0.0 ? rr / pap : 0.0; }
+
+template <typename W, int VP, int OP>
+__global__ __launch_bounds__(1024) void k_ps(PsArgs<W> A, PsGeom q, W c0, W c1, W c2, W c3) {
+  typedef PzVec<W, VP> V;
+  constexpr bool kTwo = OP == kPsFirst || OP == kPsNext1 || OP == kPsNext2;  // A applied to the formed vector too
+  constexpr bool kRho = OP == kPsRho1 || OP == kPsRho2, kFin = OP >= kPsFin2;
+  constexpr bool kS2 = OP == kPsNext2 || OP == kPsRho2 || OP == kPsFin3;
+  constexpr int RIM = kTwo ? 2 : 1, ND = OP == kPsFirst ? 3 : (kTwo ? 4 : 1);
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  __shared__ double red[16][4];
+  __shared__ double sc[4];
+  W *lds = reinterpret_cast<W *>(smem_raw);
+  // logical block: row tile fastest, then z-run, then band; the 8 XCDs each
+  // take one contiguous range, so neighbouring tiles share an L2
+  const unsigned nblk = gridDim.x, xc = blockIdx.x % 8;
+  const unsigned lb = xc * (nblk / 8) + min(xc, nblk % 8) + blockIdx.x / 8;
+  const int yt = int(lb % unsigned(q.nty)), zr = int((lb / unsigned(q.nty)) % unsigned(q.nzr));
+  const int b = int(lb / unsigned(q.nty * q.nzr)), seg = zr * q.nty + yt, nseg = q.nty * q.nzr;
+  double *S = A.scal + int64_t(b) * kPsScal;
+  if (OP == kPsFirst) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *A.above = 0;
+  } else if (threadIdx.x < 64) {
+    // finish the sums of the passes before; every block of the band finds
+    // the same values, the first one keeps them for the later passes
+    const int k = A.k;
+    const bool keep = seg == 0 && threadIdx.x == 0;
+    if (kRho) {  // a_{k-1} and <r_k, r_k>; p_{k-1}'s pass is in part_in
+      const int nd = k == 1 ? 3 : 4;
+      const double rr = ps_sum(A.part_in, b, A.nin, nd, 0), pap = ps_sum(A.part_in, b, A.nin, nd, 1);
+      const double aa = ps_sum(A.part_in, b, A.nin, nd, 2), ra = k == 1 ? pap : ps_sum(A.part_in, b, A.nin, nd, 3);
+      // with a as rounded for the update, so that the sum is that of the residual formed
+      const double a = ps_alpha(rr, pap), aw = double(W(a)), rn = rr + aw * (aw * aa - 2.0 * ra);
+      const bool direct = !(rn >= kPsGuard * rr);
+      if (threadIdx.x == 0) {
+        sc[0] = a;
+        sc[1] = k > 1 ? S[3 + k - 2] : 0.0;
+        sc[3] = direct ? 1.0 : 0.0;
+      }
+      if (keep) {
+        S[k - 1] = a;
+        S[5 + k - 1] = rr;
+        S[5 + k] = rn;
+        S[8] = direct ? 1.0 : 0.0;
+        if (k == 1 && !(rr < 1e-24)) atomicOr(A.above, 1);
+      }
+    } else if (kTwo) {  // b_{k-1}, from the direct sum where it was taken
+      const bool direct = S[8] != 0.0;
+      const double dsum = ps_sum(A.part_rho, b, direct ? A.nrho : 0, 1, 0);
+      const double rr = S[5 + k - 1], rn = direct ? dsum : S[5 + k], bt = rr != 0.0 ? rn / rr : 0.0;
+      if (threadIdx.x == 0) {
+        sc[0] = S[k - 1];
+        sc[1] = bt;
+        sc[2] = k > 1 ? S[3 + k - 2] : 0.0;
+      }
+      if (keep) S[3 + k - 1] = bt;
+    } else {  // x: the last direction's a from the sums of its pass
+      const double rr = ps_sum(A.part_in, b, A.nin, 4, 0), pap = ps_sum(A.part_in, b, A.nin, 4, 1);
+      if (threadIdx.x == 0) {
+        // every first residual below the early-exit bound: x = g
+        const bool skip = *A.above == 0;
+        sc[0] = skip ? 0.0 : ps_alpha(rr, pap);
+        sc[1] = skip ? 0.0 : S[0];
+        sc[2] = skip || OP != kPsFin3 ? 0.0 : S[1];
+      }
+    }
+  }
+  const int G = q.n1 / VP, rows = q.ty + 2 * RIM;
+  const int tid = threadIdx.x;
+  const bool act = tid < G * rows;
+  const int row = act ? tid / G : 0, x = act ? VP * (tid - row * G) : 0;
+  const int y0 = yt * q.ty, ym = y0 - RIM + row, yw = ((ym % q.n2) + q.n2) % q.n2;
+  const bool own = act && row >= RIM && row < RIM + q.ty && ym < q.n2;
+  const unsigned e0 = unsigned(x) + unsigned(yw) * unsigned(q.n1);  // offsets inside one band stay below N < 2^31
+  const unsigned n12 = unsigned(q.n12);
+  const int plane = rows * q.n1, le = row * q.n1 + x;
+  const int lu = (row + 1 < rows ? row + 1 : row) * q.n1 + x, ld = (row > 0 ? row - 1 : row) * q.n1 + x;
+  const int ll = row * q.n1 + (x == 0 ? q.n1 - 1 : x - 1), lr = row * q.n1 + (x + VP == q.n1 ? 0 : x + VP);
+  const W *s1 = A.s1 + int64_t(b) * A.ld1, *s2 = kS2 ? A.s2 + int64_t(b) * q.N : nullptr;
+  const W *gb = kFin ? A.g + int64_t(b) * q.ld : nullptr;
+  W *ob = A.out ? A.out + int64_t(b) * A.ldo : nullptr;
+  const int z0 = zr * q.zlen, z1 = min(z0 + q.zlen, q.n3);
+  auto wz = [&](int z) { return ((z % q.n3) + q.n3) % q.n3; };
+  auto ldv = [](const W *p, unsigned e) { return *reinterpret_cast<const V *>(p + e); };
+  auto stv = [](W *p, unsigned e, const V &v) { *reinterpret_cast<V *>(p + e) = v; };
+  // A applied to the plane in LDS (centre c, planes above and below hi, lo)
+  auto lap = [&](const W *pl, const V &c, const V &lo, const V &hi) {
+    const V u = *reinterpret_cast<const V *>(pl + lu), d = *reinterpret_cast<const V *>(pl + ld);
+    const W l = pl[ll], r = pl[lr];
+    V o;
+#pragma unroll
+    for (int i = 0; i < VP; ++i) {
+      const W xp = i + 1 < VP ? c.v[i + 1 < VP ? i + 1 : i] : r, xm = i > 0 ? c.v[i > 0 ? i - 1 : i] : l;
+      o.v[i] = c0 * c.v[i] + c1 * (xp + xm) + c2 * (u.v[i] + d.v[i]) + c3 * (hi.v[i] + lo.v[i]);
+    }
+    return o;
+  };
+  __syncthreads();
+  if (kRho && sc[3] == 0.0) return;  // block-uniform: the band's <r, r> is known
+  // the formed vector: r = s1 - fb s2 - fa A s1 (r_k), then p = r + fp s1
+  // (p_k; fp = 0 leaves r): the residual first, as the plain iteration forms
+  // it, so that no coefficient 1 + b is rounded
+  W fa = W(1), fb = W(0), fp = W(0), al = W(0), al1 = W(0), al2 = W(0);
+  if (OP == kPsNext1 || OP == kPsNext2) {
+    fa = W(sc[0]);
+    fb = W(sc[2]);
+    fp = W(sc[1]);
+  } else if (kRho) {
+    fa = W(sc[0]);
+    fb = W(sc[1]);
+  } else if (kFin) {
+    al = W(sc[0]);   // the last direction's
+    al1 = W(sc[1]);  // a_0
+    al2 = W(sc[2]);  // a_1
+    fa = W(S[OP == kPsFin2 ? 0 : 1]);
+    fb = W(OP == kPsFin2 ? 0.0 : S[3]);
+    fp = W(S[OP == kPsFin2 ? 3 : 4]);
+  }
+  auto form = [&](W s, W t, W as) {
+    W r = kS2 ? s - fb * t : s;
+    r = r - fa * as;
+    return OP == kPsFirst || kRho ? r : r + fp * s;
+  };
+  double acc[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) acc[d] = 0.0;
+  if constexpr (kTwo) {
+    // step zz: u(zz + 1) from the input planes zz .. zz + 2, then A u(zz)
+    V i0 = ldv(s1, unsigned(wz(z0 - 2)) * n12 + e0), i1 = ldv(s1, unsigned(wz(z0 - 1)) * n12 + e0);
+    V i2 = ldv(s1, unsigned(z0) * n12 + e0), t = V{}, um{}, u0{};
+    if (kS2) t = ldv(s2, unsigned(wz(z0 - 1)) * n12 + e0);
+    int zi = wz(z0 + 1), zt = z0;
+    for (int zz = z0 - 2; zz < z1; ++zz) {
+      W *li = lds + (zz & 1) * 2 * plane, *lq = li + plane;
+      if (act) {
+        stv(li, unsigned(le), i1);
+        stv(lq, unsigned(le), u0);
+      }
+      const V in = ldv(s1, unsigned(zi) * n12 + e0);
+      V tn{};
+      if (kS2) tn = ldv(s2, unsigned(zt) * n12 + e0);
+      zi = zi + 1 == q.n3 ? 0 : zi + 1;
+      zt = zt + 1 == q.n3 ? 0 : zt + 1;
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      const V ai = lap(li, i1, i0, i2);
+      V u1;
+#pragma unroll
+      for (int i = 0; i < VP; ++i) u1.v[i] = form(i1.v[i], t.v[i], ai.v[i]);
+      if (zz >= z0) {  // block-uniform
+        const V au = lap(lq, u0, um, u1);
+        if (own) {
+#pragma unroll
+          for (int i = 0; i < VP; ++i) {
+            const double u = double(u0.v[i]), v = double(au.v[i]);
+            const double r = OP == kPsFirst ? u : double(u0.v[i] - fp * i0.v[i]);
+            acc[0] += r * r;
+            acc[1] += u * v;
+            acc[2] += v * v;
+            if (ND > 3) acc[ND - 1] += r * v;
+          }
+          if (ob) stv(ob, unsigned(zz) * n12 + e0, u0);
+        }
+      }
+      i0 = i1;
+      i1 = i2;
+      i2 = in;
+      t = tn;
+      um = u0;
+      u0 = u1;
+    }
+  } else {
+    V i0 = ldv(s1, unsigned(wz(z0 - 1)) * n12 + e0), i1 = ldv(s1, unsigned(z0) * n12 + e0);
+    V i2 = ldv(s1, unsigned(wz(z0 + 1)) * n12 + e0), t{}, g{};
+    if (kS2) t = ldv(s2, unsigned(z0) * n12 + e0);
+    if (kFin) g = ldv(gb, unsigned(z0) * n12 + e0);
+    int zi = wz(z0 + 2), zt = wz(z0 + 1);
+    for (int z = z0; z < z1; ++z) {
+      W *li = lds + ((z - z0) & 1) * plane;
+      if (act) stv(li, unsigned(le), i1);
+      const V in = ldv(s1, unsigned(zi) * n12 + e0);
+      V tn{}, gn{};
+      if (kS2) tn = ldv(s2, unsigned(zt) * n12 + e0);
+      if (kFin) gn = ldv(gb, unsigned(zt) * n12 + e0);
+      zi = zi + 1 == q.n3 ? 0 : zi + 1;
+      zt = zt + 1 == q.n3 ? 0 : zt + 1;
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      const V ai = lap(li, i1, i0, i2);
+      if (own) {
+        V xo;
+#pragma unroll
+        for (int i = 0; i < VP; ++i) {
+          const W v = form(i1.v[i], t.v[i], ai.v[i]);
+          if (kRho) {
+            acc[0] += double(v) * double(v);
+          } else {
+            const W gv = g.v[i];
+            W xv = gv;
+            if (OP == kPsFin2) xv += al1 * i1.v[i];
+            if (OP == kPsFin3) xv = xv + al1 * t.v[i] + al2 * i1.v[i];
+            xv += al * v;
+            xo.v[i] = xv;
+            acc[0] += double(xv) * double(gv);
+          }
+        }
+        if (kFin) stv(ob, unsigned(z) * n12 + e0, xo);
+      }
+      i0 = i1;
+      i1 = i2;
+      i2 = in;
+      t = tn;
+      g = gn;
+    }
+  }
+  const int lane = tid & 63, wid = tid >> 6, nw = (blockDim.x + 63) >> 6;
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    double v = acc[d];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (lane == 0) red[wid][d] = v;
+  }
+  __syncthreads();
+  if (tid < ND) {
+    double v = 0.0;
+    for (int k = 0; k < nw; ++k) v += red[k][tid];
+    A.part[(int64_t(b) * nseg + seg) * ND + tid] = v;
+  }
+}
+
 // A <- s (A + A^T) in place (both triangles), for an n x n matrix
 __global__ void k_symmetrize(double *__restrict__ A, int n, double s) {
   const int i = blockIdx.x * 16 + threadIdx.x, j = blockIdx.y * 16 + threadIdx.y;
@@ -901,8 +1195,7 @@ int multidot_t(rsg_ctx *ctx, int npair, const W *const *x, const W *const *y, in
 #undef RSG_DOT_CASE
   }
   const int count = npair * nb;
-  hipLaunchKernelGGL(k_reduce_partials, dim3((count + 255) / 256), dim3(256), 0, ctx->stream, partial,
-                     nseg, count, alpha, out);
+  reduce_partials(ctx, partial, nseg, count, alpha, out);
   return RSG_OK;
 }
 
@@ -928,8 +1221,7 @@ int ritz_dots(rsg_ctx *ctx, const W *x, const W *p, const W *hx, const W *hp, in
   hipLaunchKernelGGL((k_ritz_dots<W>), dim3(nseg, nb), dim3(kThreads), 0, ctx->stream, x, p, hx, hp, N, nb, nseg,
                      seglen, partial);
   const int count = 6 * nb;
-  hipLaunchKernelGGL(k_reduce_partials, dim3((count + 255) / 256), dim3(256), 0, ctx->stream, partial, nseg, count,
-                     alpha, out);
+  reduce_partials(ctx, partial, nseg, count, alpha, out);
   return RSG_OK;
 }
 
@@ -1008,6 +1300,94 @@ int precond_hprsdft(rsg_ctx *ctx, int mloop, const W *g, W *pg, int nn, W *r, W 
 }
 
 
+// Rows per block and z-runs of a k_ps pass: the fewest rounds of blocks over
+// the chip, times the planes a block walks (its run and the rim), times the
+// cost of a plane (never below the latency of one step).  False where a row
+// does not leave room for at least four tile rows.
+bool ps_geom(const rsg_ctx *ctx, int vp, size_t wsize, int rim, int nn, int64_t ld, PsGeom &q) {
+  const int n1 = ctx->n[0], n2 = ctx->n[1], n3 = ctx->n[2], G = n1 / vp;
+  const int narr = rim == 2 ? 4 : 2;
+  double best = 1e300;
+  for (int nty = 1; nty <= std::max(1, n2 / 4); ++nty) {
+    const int ty = (n2 + nty - 1) / nty, rows = ty + 2 * rim, th = (G * rows + 63) / 64 * 64;
+    if (th > 1024 || size_t(narr) * rows * n1 * wsize > 63 * 1024) continue;
+    const int per_cu = std::max(1, std::min(4, 1024 / th));
+    for (int nzr : {1, 2, 3, 4, 6, 8, 12, 16, 24}) {
+      if (nzr > 1 && nzr > n3 / 4) break;
+      const int zlen = (n3 + nzr - 1) / nzr;
+      const double rounds = std::ceil(double(nty) * nzr * nn / (256.0 * per_cu));
+      const double cost = rounds * (zlen + 2 * rim) * std::max(0.45, per_cu * th / 1024.0);
+      if (cost < best) {
+        best = cost;
+        q.ty = ty;
+        q.nty = (n2 + ty - 1) / ty;
+        q.zlen = zlen;
+      }
+    }
+  }
+  if (best > 1e299) return false;
+  q.n1 = n1;
+  q.n2 = n2;
+  q.n3 = n3;
+  q.N = ctx->N;
+  q.n12 = int64_t(n1) * n2;
+  q.ld = ld;
+  q.nzr = (n3 + q.zlen - 1) / q.zlen;
+  return int64_t(q.nty) * q.nzr * nn <= 0x7fffffff;
+}
+
+// The recomputing passes (k_ps) for mloop 2 or 3: pg = P g and rb = dv <pg,
+// g>; r and p take p_0 and p_1.  q2 / q1: geometry of the passes with a rim
+// of two / one rows.
+template <typename W, int VP>
+int precond_ps(rsg_ctx *ctx, int mloop, const W *g, W *pg, int nn, W *r, W *p, Scratch &s, double dv, double *rb,
+               const PsGeom &q2, const PsGeom &q1, W C0, W C1, W C2, W C3) {
+  const int n2 = q2.nty * q2.nzr, n1 = q1.nty * q1.nzr;  // blocks, so partial sums, per band
+  // partial sums: two passes of up to 4 products, one of <r, r> / <x, g>; scalars per band
+  const size_t o2 = 4 * size_t(nn) * n2, o1 = size_t(nn) * n1;
+  if (ctx->dotpart.ensure((2 * o2 + o1 + size_t(nn) * kPsScal) * sizeof(double)) != hipSuccess)
+    return ctx->fail(RSG_ERR_HIP, "preconditioner: scratch allocation failed");
+  double *pa = ctx->dotpart.as<double>(), *pb = pa + o2, *pr = pb + o2, *sc = pr + o1;
+  const int G = q2.n1 / VP;
+  auto pass = [&](auto opc, const W *s1, int64_t ld1, const W *s2, W *out, const double *in, double *part, int k) {
+    constexpr int OP = decltype(opc)::value;
+    constexpr bool two = OP == kPsFirst || OP == kPsNext1 || OP == kPsNext2;
+    const PsGeom &q = two ? q2 : q1;
+    PsArgs<W> A{};
+    A.s1 = s1;
+    A.s2 = s2;
+    A.g = g;
+    A.out = out;
+    A.ld1 = ld1;
+    A.ldo = OP >= kPsFin2 ? q.ld : q.N;
+    A.part_in = in;
+    A.part_rho = pr;
+    A.part = part;
+    A.scal = sc;
+    A.nin = n2;
+    A.nrho = n1;
+    A.k = k;
+    A.above = s.flags + 1;
+    const int rows = q.ty + (two ? 4 : 2), th = (G * rows + 63) / 64 * 64;
+    const size_t lds = size_t(two ? 4 : 2) * rows * q.n1 * sizeof(W);
+    hipLaunchKernelGGL((k_ps<W, VP, OP>), dim3(unsigned(int64_t(q.nty) * q.nzr * nn)), dim3(th), lds, ctx->stream, A,
+                       q, C0, C1, C2, C3);
+  };
+  pass(std::integral_constant<int, kPsFirst>{}, g, q2.ld, nullptr, r, nullptr, pa, 0);
+  pass(std::integral_constant<int, kPsRho1>{}, r, q2.N, nullptr, nullptr, pa, pr, 1);
+  pass(std::integral_constant<int, kPsNext1>{}, r, q2.N, nullptr, mloop == 2 ? nullptr : p, nullptr, pb, 1);
+  if (mloop == 2) {
+    pass(std::integral_constant<int, kPsFin2>{}, r, q2.N, nullptr, pg, pb, pr, 1);
+  } else {
+    pass(std::integral_constant<int, kPsRho2>{}, p, q2.N, r, nullptr, pb, pr, 2);
+    pass(std::integral_constant<int, kPsNext2>{}, p, q2.N, r, nullptr, nullptr, pa, 2);
+    pass(std::integral_constant<int, kPsFin3>{}, p, q2.N, r, pg, pa, pr, 2);
+  }
+  reduce_partials(ctx, pr, n1, nn, dv, rb);
+  RSG_HIP(hipGetLastError());
+  return RSG_OK;
+}
+
 // precond_hprsdft in z-streaming passes for the CG step (no diagonal
 // shift): pg = P g and rb = dv <pg, g>.  The same iteration as
 // precond_hprsdft; f is the second direction buffer.
@@ -1047,6 +1427,17 @@ int precond_hprsdft_fused(rsg_ctx *ctx, int mloop, const W *g, W *pg, int nn, W 
            reinterpret_cast<uintptr_t>(pg) % va == 0;
   };
   const int vp = (sizeof(W) == 4 && fits(4)) ? 4 : (fits(2) ? 2 : 1);
+  // two or three steps: the recomputing passes, where a block holds enough rows
+  if ((mloop == 2 || mloop == 3) && !(sizeof(W) == 4 && ctx->pc_bf16 && vp >= 2)) {
+    PsGeom q2, q1;
+    if (ps_geom(ctx, vp, sizeof(W), 2, nn, ld, q2) && ps_geom(ctx, vp, sizeof(W), 1, nn, ld, q1)) {
+      if constexpr (sizeof(W) == 4) {
+        if (vp == 4) return precond_ps<W, 4>(ctx, mloop, g, pg, nn, r, p, s, dv, rb, q2, q1, C0, C1, C2, C3);
+      }
+      if (vp == 2) return precond_ps<W, 2>(ctx, mloop, g, pg, nn, r, p, s, dv, rb, q2, q1, C0, C1, C2, C3);
+      return precond_ps<W, 1>(ctx, mloop, g, pg, nn, r, p, s, dv, rb, q2, q1, C0, C1, C2, C3);
+    }
+  }
   q.nq = int((q.n12 / vp + kThreads - 1) / kThreads);
   // enough blocks to fill the chip; z-runs of at least 4 planes
   const int64_t per_run = int64_t(q.nq) * nn;
@@ -1073,9 +1464,8 @@ int precond_hprsdft_fused(rsg_ctx *ctx, int mloop, const W *g, W *pg, int nn, W 
     A.rr0 = s.rr0;
     A.partial = ctx->dotpart.as<double>();
     const dim3 grid(unsigned(int64_t(q.nseg) * nn)), blk(kThreads), gb((nn + 63) / 64), b64(64);
-    const dim3 gr((nn + 255) / 256);
     auto reduce = [&](double alpha, double *out) {
-      hipLaunchKernelGGL(k_reduce_partials, gr, dim3(256), 0, ctx->stream, A.partial, q.nseg, nn, alpha, out);
+      reduce_partials(ctx, A.partial, q.nseg, nn, alpha, out);
     };
     auto pass = [&](auto opc) {
       constexpr int OP = decltype(opc)::value;

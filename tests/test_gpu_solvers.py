@@ -537,3 +537,38 @@ def test_conjugate_gradient_graph_replays_equal_direct_launches(setup, precision
         assert ctx.cg_graph_launches() - n0 >= 3  # captured once, then replayed
     finally:
         ctx.set_cg_graphs(False)
+
+
+@pytest.mark.parametrize("ngrid", [(36, 36, 36), (45, 14, 11), (24, 5, 30)])
+@pytest.mark.parametrize("mloop", [2, 3])
+def test_precond_hprsdft_near_eigenvectors(orc, ngrid, mloop):
+    """Bands whose residual nearly vanishes after one step (a plane wave, and
+    two plane waves of close eigenvalues), where <r, r> is summed directly
+    instead of from the previous pass, beside ordinary, zero and tiny bands.
+    FP64 against the oracle: 1e-12 of each band's largest value."""
+    import dataclasses
+
+    from rsdft_develop_amd import gpu
+
+    cell = dataclasses.replace(systems.silicon_supercell(1, nband=4), ngrid=ngrid)
+    ham = orc.Ham(cell, vloc=None, projectors=False)
+    ctx = gpu.Context()
+    ctx.set_grid(cell.ngrid, cell.aa, cell.md)
+    N = cell.npoints
+    z, y, x = np.meshgrid(*(2 * np.pi * np.arange(n) / n for n in ngrid[::-1]), indexing="ij")
+    rng = np.random.default_rng(11)
+    g = np.zeros((N, 6))
+    g[:, 0] = np.cos(3 * x).ravel()
+    g[:, 1] = (np.cos(2 * x) + 0.3 * np.sin(2 * y + x)).ravel()
+    g[:, 2] = rng.standard_normal(N)
+    g[:, 4] = 1e-9 * rng.standard_normal(N)
+    g[:, 5] = (np.sin(z) + 1e-3 * np.cos(4 * x)).ravel()
+    want = ham.precond(g, mloop=mloop)
+    print(f"case: precond near eigenvectors {ngrid} mloop {mloop}", flush=True)
+    got = _precond_gpu(ctx, g, N, mloop, np.float64)
+    for b in range(g.shape[1]):
+        if not g[:, b].any():
+            assert not got[:, b].any()
+            continue
+        err = np.abs(got[:, b] - want[:, b]).max() / np.abs(want[:, b]).max()
+        assert err <= 1e-12, (b, err)
