@@ -172,6 +172,7 @@ struct HpsiShape {
 struct LpcState {
   DevBuf wbf, bias, vnorm, x0, a1, a2, y, dyb, dz1, dz2, sval, gg, part, grad, master, mom1, mom2, lsum;
   DevBuf diag, tbuf;  // training-target solve
+  DevBuf xq, dq;      // quad layouts of a layer's input and output gradient (weight gradients)
   bool have_params = false, have_v = false;
   int64_t vN = 0;
   int adam_t = 0;

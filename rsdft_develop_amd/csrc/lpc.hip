@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "lpc.hpp"
@@ -35,7 +36,6 @@ typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 4;  // waves per workgroup in the convolution kernels
-constexpr int kTiles = 4;  // 16-point tiles per wave
 
 __host__ __device__ inline uint16_t f2bf(float f) {
   uint32_t u;
@@ -55,46 +55,19 @@ struct Grid3 {
   int n1, n2, n3;
 };
 
-// neighbour of point (i1, i2, i3) at tap t (offsets d - 1 in {-1, 0, 1})
-__device__ inline int64_t nbr(const Grid3 &g, int i1, int i2, int i3, int t) {
-  const int d3 = t / 9, d2 = (t / 3) % 3, d1 = t % 3;
-  int x = i1 + d1 - 1, y = i2 + d2 - 1, z = i3 + d3 - 1;
-  x = x < 0 ? x + g.n1 : (x >= g.n1 ? x - g.n1 : x);
-  y = y < 0 ? y + g.n2 : (y >= g.n2 ? y - g.n2 : y);
-  z = z < 0 ? z + g.n3 : (z >= g.n3 ? z - g.n3 : z);
-  return x + int64_t(g.n1) * (y + int64_t(g.n2) * z);
+__device__ inline bf16x4 as_bf16x4(uint2 w) {
+  bf16x4 v;
+  v[0] = short(w.x & 0xffff);
+  v[1] = short(w.x >> 16);
+  v[2] = short(w.y & 0xffff);
+  v[3] = short(w.y >> 16);
+  return v;
 }
 
-// B fragment of chunk c for the lane's point: X[k][p], k = 16c + 4(l/16) + i
-template <int CIN>
-__device__ inline bf16x4 load_b(const uint16_t *__restrict__ in, const Grid3 &g, int i1, int i2, int i3, int c,
-                                int lq) {
-  bf16x4 v;
-  if constexpr (CIN == 16) {
-    const int64_t q = nbr(g, i1, i2, i3, c);
-    const uint2 w = *reinterpret_cast<const uint2 *>(in + q * 16 + 4 * lq);
-    v[0] = short(w.x & 0xffff);
-    v[1] = short(w.x >> 16);
-    v[2] = short(w.y & 0xffff);
-    v[3] = short(w.y >> 16);
-  } else if constexpr (CIN == 2) {
-    const int t0 = (16 * c + 4 * lq) / 2;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int t = t0 + h;
-      uint32_t w = 0;
-      if (t < 27) w = *reinterpret_cast<const uint32_t *>(in + nbr(g, i1, i2, i3, t) * 2);
-      v[2 * h] = short(w & 0xffff);
-      v[2 * h + 1] = short(w >> 16);
-    }
-  } else {  // CIN == 1
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = 16 * c + 4 * lq + i;
-      v[i] = t < 27 ? short(in[nbr(g, i1, i2, i3, t)]) : short(0);
-    }
-  }
-  return v;
+// i + d - 1 on an axis of n points, periodic
+__device__ inline int tap_wrap(int i, int d, int n) {
+  const int j = i + d - 1;
+  return j < 0 ? j + n : (j >= n ? j - n : j);
 }
 
 enum ConvMode { kReluOut = 0, kFinalOut = 1, kMaskedGrad = 2 };
@@ -104,73 +77,164 @@ enum ConvMode { kReluOut = 0, kFinalOut = 1, kMaskedGrad = 2 };
 //  kFinalOut:  y = D[0] + bias[0]; yout[p] = y (FP32 if non-null);
 //              pg[p] = s y  (the preconditioned residual, type T)
 //  kMaskedGrad: out_bf[p][co] = bf16(D * (mask[p][co] > 0))    (16 outputs)
+//
+// A wave owns 16 consecutive points of an xy-plane of one sample and walks
+// a run of z-planes.  The in-plane offsets of its neighbours are the same
+// in every plane, so they are formed once.  With 16 input channels (a K
+// chunk of 16 is one tap) the nine fragments of a plane serve the three
+// output planes it touches: it is the d3 = 2 tap plane of the output below,
+// d3 = 1 of its own and d3 = 0 of the output above, each with its own
+// accumulators.  9 loads feed 27 products, where a gather of each tap took
+// 27 loads and their address arithmetic.  Three accumulator chains per
+// output (taps c mod 3, that is d1): one chain's latency would bound the
+// tile.  With one or two input channels a lane's K slots are different
+// taps, loaded for each output plane.
 template <int CIN, int KP, int MODE, typename T>
-__global__ __launch_bounds__(64 * kWaves) void k_conv(Grid3 g, int64_t N, const uint16_t *__restrict__ in,
-                                                      int64_t in_stride, const uint16_t *__restrict__ wbf,
+__global__ __launch_bounds__(64 * kWaves) void k_conv(Grid3 g, int64_t N, int zlen, int nzr, int ntg,
+                                                      const uint16_t *__restrict__ in, int64_t in_stride,
+                                                      const uint16_t *__restrict__ wbf,
                                                       const float *__restrict__ bias, uint16_t *__restrict__ out_bf,
                                                       const uint16_t *__restrict__ mask, float *__restrict__ yout,
-                                                      const T *__restrict__ gsrc, T *__restrict__ pg, int64_t ldg,
+                                                      T *__restrict__ pg, int64_t ldg,
                                                       const float *__restrict__ sval) {
   constexpr int NC = KP / 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lq = lane >> 4, lr = lane & 15;
-  const int smp = blockIdx.y;
+  // logical block: tile group fastest, then z-run, then sample; each XCD
+  // takes one contiguous range, so neighbouring tiles share an L2
+  const unsigned nblk = gridDim.x, xc = blockIdx.x % 8;
+  const unsigned lb = xc * (nblk / 8) + min(xc, nblk % 8) + blockIdx.x / 8;
+  const int tg = int(lb % unsigned(ntg)), zr = int((lb / unsigned(ntg)) % unsigned(nzr));
+  const int smp = int(lb / unsigned(ntg * nzr));
+  const int n12 = g.n1 * g.n2, j0 = (tg * kWaves + wave) * 16;
+  if (j0 >= n12) return;  // whole wave; no barriers in this kernel
   const uint16_t *__restrict__ src = in + int64_t(smp) * in_stride;
+  const int j = min(j0 + lr, n12 - 1), x = j % g.n1, y = j / g.n1;
+  const bool ok = j0 + lr < n12;
+  const int z0 = zr * zlen, z1 = min(z0 + zlen, g.n3);
   // A fragments: W[co = lr][k = 16c + 4 lq + i]
   bf16x4 a[NC];
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const uint2 w = *reinterpret_cast<const uint2 *>(wbf + lr * KP + 16 * c + 4 * lq);
-    a[c][0] = short(w.x & 0xffff);
-    a[c][1] = short(w.x >> 16);
-    a[c][2] = short(w.y & 0xffff);
-    a[c][3] = short(w.y >> 16);
-  }
-  const int64_t base = (int64_t(blockIdx.x) * kWaves + wave) * (16 * kTiles);
-  for (int t = 0; t < kTiles; ++t) {
-    const int64_t p0 = base + 16 * t;
-    if (p0 >= N) break;  // wave-uniform
-    const int64_t p = min(p0 + lr, N - 1);
-    const int i1 = int(p % g.n1), i2 = int((p / g.n1) % g.n2), i3 = int(p / (int64_t(g.n1) * g.n2));
-    // three independent accumulator chains (taps c mod 3): the matrix-core
-    // latency of one chain of NC dependent products, not its issue rate,
-    // would otherwise bound the tile
-    f32x4 acc3[3] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  for (int c = 0; c < NC; ++c) a[c] = as_bf16x4(*reinterpret_cast<const uint2 *>(wbf + lr * KP + 16 * c + 4 * lq));
+  float bs[4] = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (MODE == kReluOut) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const bf16x4 b = load_b<CIN>(src, g, i1, i2, i3, c, lq);
-      acc3[c % 3] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[c], b, acc3[c % 3], 0, 0, 0);
-    }
+    for (int i = 0; i < 4; ++i) bs[i] = bias[4 * lq + i];
+  }
+  const float b0 = MODE == kFinalOut ? bias[0] : 0.f;
+  auto finish = [&](int z, const f32x4 (&acc3)[3]) {
     const f32x4 acc = (acc3[0] + acc3[1]) + acc3[2];
-    const bool ok = p0 + lr < N;
+    const int64_t p = int64_t(z) * n12 + j;
     if constexpr (MODE == kReluOut || MODE == kMaskedGrad) {
+      const int64_t o = int64_t(smp) * N * 16 + p * 16 + 4 * lq;
       uint16_t h[4];
+      bf16x4 m{};
+      if constexpr (MODE == kMaskedGrad) m = as_bf16x4(*reinterpret_cast<const uint2 *>(mask + o));
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int co = 4 * lq + i;
-        float z = acc[i];
+        float v = acc[i];
         if constexpr (MODE == kReluOut) {
-          z += bias[co];
-          z = z > 0.f ? z : 0.f;
+          v += bs[i];
+          v = v > 0.f ? v : 0.f;
         } else {
-          const uint16_t m = mask[int64_t(smp) * N * 16 + p * 16 + co];
-          z = bf2f(m) > 0.f ? z : 0.f;
+          v = bf2f(uint16_t(m[i])) > 0.f ? v : 0.f;
         }
-        h[i] = f2bf(z);
+        h[i] = f2bf(v);
       }
       if (ok) {
         uint2 w;
         w.x = uint32_t(h[0]) | (uint32_t(h[1]) << 16);
         w.y = uint32_t(h[2]) | (uint32_t(h[3]) << 16);
-        *reinterpret_cast<uint2 *>(out_bf + int64_t(smp) * N * 16 + p * 16 + 4 * lq) = w;
+        *reinterpret_cast<uint2 *>(out_bf + o) = w;
       }
     } else {
       // row co = 0 lives in acc[0] of lanes 0..15
       if (lq == 0 && ok) {
-        const float y = acc[0] + bias[0];
-        if (yout) yout[int64_t(smp) * N + p] = y;
-        if (pg) pg[int64_t(smp) * ldg + p] = T(double(sval[smp]) * double(y));
+        const float yv = acc[0] + b0;
+        if (yout) yout[int64_t(smp) * N + p] = yv;
+        if (pg) pg[int64_t(smp) * ldg + p] = T(double(sval[smp]) * double(yv));
       }
+    }
+  };
+  if constexpr (CIN == 16) {
+    int ofs[9];
+#pragma unroll
+    for (int t = 0; t < 9; ++t) ofs[t] = (tap_wrap(x, t % 3, g.n1) + g.n1 * tap_wrap(y, t / 3, g.n2)) * 16 + 4 * lq;
+    const int64_t pstr = int64_t(n12) * 16;
+    f32x4 acc[3][3];  // [output plane mod 3][chain]
+    uint2 nf[9];
+    int zn = z0 == 0 ? g.n3 - 1 : z0 - 1;  // input plane to fetch
+    auto fetch = [&]() {
+      const uint16_t *sp = src + zn * pstr;
+#pragma unroll
+      for (int t = 0; t < 9; ++t) nf[t] = *reinterpret_cast<const uint2 *>(sp + ofs[t]);
+      zn = zn + 1 == g.n3 ? 0 : zn + 1;
+    };
+    fetch();
+    // step s: input plane z0 - 1 + s; U = s mod 3 is the slot of output s (plane z0 + s)
+    auto step = [&](int s, auto uc) {
+      constexpr int U = decltype(uc)::value, Um1 = (U + 2) % 3, Um2 = (U + 1) % 3;
+      uint2 f[9];
+#pragma unroll
+      for (int t = 0; t < 9; ++t) f[t] = nf[t];
+      if (s + 1 < z1 - z0 + 2) fetch();
+#pragma unroll
+      for (int d = 0; d < 3; ++d) acc[U][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 9; ++t) {
+        const bf16x4 b = as_bf16x4(f[t]);
+        acc[U][t % 3] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[t], b, acc[U][t % 3], 0, 0, 0);
+        acc[Um1][t % 3] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[9 + t], b, acc[Um1][t % 3], 0, 0, 0);
+        acc[Um2][t % 3] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[18 + t], b, acc[Um2][t % 3], 0, 0, 0);
+      }
+      if (s >= 2) finish(z0 + s - 2, acc[Um2]);  // outputs s - 2 >= 0 are complete
+    };
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) acc[u][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int ns = z1 - z0 + 2;
+    for (int s = 0; s < ns; s += 3) {
+      step(s, std::integral_constant<int, 0>{});
+      if (s + 1 < ns) step(s + 1, std::integral_constant<int, 1>{});
+      if (s + 2 < ns) step(s + 2, std::integral_constant<int, 2>{});
+    }
+  } else {
+    // K slot k = 16 c + 4 lq + i is channel k % CIN of tap k / CIN: the
+    // lane's taps, their in-plane offsets and planes
+    constexpr int NT = NC * 4 / CIN;
+    int ofs[NT], dz[NT];
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      const int t = (16 * (u / (4 / CIN)) + 4 * lq) / CIN + u % (4 / CIN), tc = min(t, 26);
+      dz[u] = t < 27 ? tc / 9 : 3;  // 3: no tap
+      ofs[u] = (tap_wrap(x, tc % 3, g.n1) + g.n1 * tap_wrap(y, (tc / 3) % 3, g.n2)) * CIN;
+    }
+    const int64_t pstr = int64_t(n12) * CIN;
+    for (int z = z0; z < z1; ++z) {
+      const uint16_t *s0 = src + tap_wrap(z, 0, g.n3) * pstr, *s1 = src + z * pstr, *s2 = src + tap_wrap(z, 2, g.n3) * pstr;
+      f32x4 acc3[3] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+      uint32_t w[NT];
+#pragma unroll
+      for (int u = 0; u < NT; ++u) {
+        const uint16_t *p = (dz[u] == 0 ? s0 : (dz[u] == 2 ? s2 : s1)) + ofs[u];
+        if constexpr (CIN == 2)
+          w[u] = *reinterpret_cast<const uint32_t *>(p);
+        else
+          w[u] = *p;
+      }
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        bf16x4 b;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int u = (4 / CIN) * c + i / CIN;
+          const uint32_t v = dz[u] == 3 ? 0u : (CIN == 2 && (i & 1) ? w[u] >> 16 : w[u]);
+          b[i] = short(v & 0xffff);
+        }
+        acc3[c % 3] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[c], b, acc3[c % 3], 0, 0, 0);
+      }
+      finish(z, acc3);
     }
   }
 }
@@ -217,89 +281,161 @@ __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ tgt, con
   if (threadIdx.x == 0) atomicAdd(lsum, (red[0] + red[1] + red[2] + red[3]) * inv_count);
 }
 
-// dW[co][k] += sum_p dz[p][co] X[k][p]: MFMA with co x k-chunk outputs and
-// 16 points per product.  Each workgroup folds its partial into part[blk].
+// Quad layout of a channel-last field for products that contract over the
+// points: out[row][quad][channel][4 points], a row being one x-line of one
+// sample.  Quad q holds the points x = 4 (q - 1) .. 4 (q - 1) + 3, so each
+// line has a quad in front of it; with wrap the points x = -1 and x = n1
+// are the periodic copies, everything else outside 0..n1-1 is zero.
+template <int C>
+__global__ __launch_bounds__(256) void k_quads(const uint16_t *__restrict__ in, int64_t nrow, int n1, int nq, int wrap,
+                                               uint16_t *__restrict__ out) {
+  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t >= nrow * nq * C) return;
+  const int c = int(t % C), q = int((t / C) % nq);
+  const int64_t row = t / (int64_t(C) * nq);
+  uint16_t v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int x = 4 * (q - 1) + i;
+    if (wrap && x == -1) x = n1 - 1;
+    else if (wrap && x == n1) x = 0;
+    v[i] = x >= 0 && x < n1 ? in[(row * n1 + x) * C + c] : uint16_t(0);
+  }
+  uint2 w;
+  w.x = uint32_t(v[0]) | (uint32_t(v[1]) << 16);
+  w.y = uint32_t(v[2]) | (uint32_t(v[3]) << 16);
+  *reinterpret_cast<uint2 *>(out + 4 * t) = w;
+}
+
+// dW[co][k] += sum_p dz[p][co] X[k][p], k = tap * CIN + ci, on MFMA with
+// co x 16-k-chunk outputs and 16 points of an x-line per product.  Both
+// operands hold four consecutive points of one channel per lane, so they
+// are read from the quad layout, 512 contiguous bytes a wave; the taps with
+// d1 = -1 and +1 shift the quad by one point with the quad beside it.  (A
+// gather of single channels from the channel-last fields took 2-byte loads,
+// 108 of them per lane and 16 points: 920 us against 75 us here for 16
+// samples of 36^3 points.)  Lines past n1 are zero in dz.  A wave takes
+// every (4 blocks)-th line; a block adds its four waves in order into part.
 template <int CIN, int KP, int COUT>
-__global__ __launch_bounds__(256) void k_conv_dw(Grid3 g, int64_t N, int nsamp, const uint16_t *__restrict__ in,
-                                                 const uint16_t *__restrict__ dz, int64_t pts_per_block,
-                                                 float *__restrict__ part) {
+__global__ __launch_bounds__(256) void k_conv_dw(Grid3 g, int nsamp, const uint16_t *__restrict__ xq,
+                                                 const uint16_t *__restrict__ dq, int nq, float *__restrict__ part) {
   constexpr int NC = KP / 16;
   __shared__ float red[16 * KP];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lq = lane >> 4, lr = lane & 15;
-  for (int i = threadIdx.x; i < 16 * KP; i += blockDim.x) red[i] = 0.f;
-  __syncthreads();
   f32x4 acc[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int64_t total = N * nsamp;
-  const int64_t b0 = int64_t(blockIdx.x) * pts_per_block;
-  const int64_t b1 = min(total, b0 + pts_per_block);
-  for (int64_t q0 = b0 + 16 * wave; q0 < b1; q0 += 16 * 4) {
-    // A: dz^T [co = lr][point 4 lq + i]; B: X [k = 16c + lr][point 4 lq + i]
-    bf16x4 av;
-    int smp[4], c1[4], c2[4], c3[4];
-    bool ok[4];
+  const int n23 = g.n2 * g.n3, nrow = n23 * nsamp, nch = (g.n1 + 15) / 16;
+  for (int row = blockIdx.x * 4 + wave; row < nrow; row += 4 * gridDim.x) {
+    const int smp = row / n23, zy = row - smp * n23, z = zy / g.n2, y = zy - z * g.n2;
+    int rz[3], ry[3];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t q = q0 + 4 * lq + i;
-      ok[i] = q < b1;
-      const int64_t qq = ok[i] ? q : b0;
-      smp[i] = int(qq / N);
-      const int64_t p = qq - int64_t(smp[i]) * N;
-      c1[i] = int(p % g.n1);
-      c2[i] = int((p / g.n1) % g.n2);
-      c3[i] = int(p / (int64_t(g.n1) * g.n2));
-      av[i] = (ok[i] && lr < COUT) ? short(dz[(int64_t(smp[i]) * N + p) * COUT + lr]) : short(0);
+    for (int d = 0; d < 3; ++d) {
+      const int zz = z + d - 1, yy = y + d - 1;
+      rz[d] = smp * n23 + g.n2 * (zz < 0 ? zz + g.n3 : (zz >= g.n3 ? zz - g.n3 : zz));
+      ry[d] = yy < 0 ? yy + g.n2 : (yy >= g.n2 ? yy - g.n2 : yy);
     }
+    for (int ch = 0; ch < nch; ++ch) {
+      const int qa = 1 + 4 * ch + lq;
+      bf16x4 av = {0, 0, 0, 0};
+      if (lr < COUT) av = as_bf16x4(*reinterpret_cast<const uint2 *>(dq + ((int64_t(row) * nq + qa) * COUT + lr) * 4));
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int k = 16 * c + lr;
-      const int tap = k / CIN, ci = k % CIN;
-      bf16x4 bv;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bv[i] = (ok[i] && tap < 27)
-                    ? short(in[(int64_t(smp[i]) * N + nbr(g, c1[i], c2[i], c3[i], tap)) * CIN + ci])
-                    : short(0);
+      for (int c = 0; c < NC; ++c) {
+        // CIN = 16: the chunk is one tap, the same for every lane
+        const int k = 16 * c + lr, tap = CIN == 16 ? c : min(k / CIN, 26), ci = CIN == 16 ? lr : k % CIN;
+        const int d3 = tap / 9, d2 = (tap / 3) % 3, d1 = tap % 3;
+        const int64_t r = (d3 == 0 ? rz[0] : (d3 == 1 ? rz[1] : rz[2])) + (d2 == 0 ? ry[0] : (d2 == 1 ? ry[1] : ry[2]));
+        const uint16_t *p = xq + ((r * nq + qa) * CIN + ci) * 4;
+        const uint2 w = *reinterpret_cast<const uint2 *>(p);
+        // the point before the quad, or the one after it (the middle tap reads its own quad again)
+        const uint32_t o = p[d1 == 0 ? 3 - 4 * CIN : (d1 == 2 ? 4 * CIN : 0)];
+        uint2 v = w;
+        if (d1 == 0) {
+          v.x = o | (w.x << 16);
+          v.y = (w.x >> 16) | (w.y << 16);
+        } else if (d1 == 2) {
+          v.x = (w.x >> 16) | (w.y << 16);
+          v.y = (w.y >> 16) | (o << 16);
+        }
+        if (CIN != 16 && k / CIN > 26) v.x = v.y = 0;
+        acc[c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, as_bf16x4(v), acc[c], 0, 0, 0);
       }
-      acc[c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[c], 0, 0, 0);
     }
   }
   // D[co = 4 lq + i][k = 16c + lr]
+  for (int w = 0; w < 4; ++w) {
+    if (wave == w) {
 #pragma unroll
-  for (int c = 0; c < NC; ++c)
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) atomicAdd(&red[(4 * lq + i) * KP + 16 * c + lr], acc[c][i]);
-  __syncthreads();
+        for (int i = 0; i < 4; ++i) {
+          float &o = red[(4 * lq + i) * KP + 16 * c + lr];
+          o = w == 0 ? acc[c][i] : o + acc[c][i];
+        }
+    }
+    __syncthreads();
+  }
   for (int i = threadIdx.x; i < 16 * KP; i += blockDim.x) part[int64_t(blockIdx.x) * 16 * KP + i] = red[i];
 }
 
-__global__ void k_sum_parts(const float *__restrict__ part, int nblk, int len, float *__restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= len) return;
+// out[i] = sum over nblk partial rows of len values: 64 columns a block,
+// each of its 16 waves every 16th row, the waves added in order
+__global__ __launch_bounds__(1024) void k_sum_parts(const float *__restrict__ part, int nblk, int len,
+                                                    float *__restrict__ out) {
+  __shared__ double red[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
   double s = 0.0;
-  for (int b = 0; b < nblk; ++b) s += part[int64_t(b) * len + i];
-  out[i] = float(s);
+  if (i < len)
+    for (int b = wave; b < nblk; b += 16) s += part[int64_t(b) * len + i];
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && i < len) {
+    for (int w = 1; w < 16; ++w) s += red[w][lane];
+    out[i] = float(s);
+  }
 }
 
-// bias gradient: db[co] = sum_p dz[p][co] (COUT channels, bf16)
+// bias gradient: per block sum_p dz[p][co] (COUT channels, bf16) into part[block][COUT].  A
+// thread reads eight channels (16 bytes) of a point at a time, or eight
+// points where COUT is 1, neighbouring threads neighbouring words; the
+// last words of a COUT = 1 field may hold fewer than eight points.
 template <int COUT>
 __global__ __launch_bounds__(256) void k_bias_grad(const uint16_t *__restrict__ dz, int64_t total,
-                                                   float *__restrict__ db) {
-  float acc[COUT];
+                                                   float *__restrict__ part) {
+  constexpr int H = COUT == 16 ? 2 : 1;  // words per point group
+  __shared__ float red[4][16];
+  float acc[8];
 #pragma unroll
-  for (int c = 0; c < COUT; ++c) acc[c] = 0.f;
-  for (int64_t q = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; q < total; q += int64_t(gridDim.x) * blockDim.x)
+  for (int c = 0; c < 8; ++c) acc[c] = 0.f;
+  const int64_t nval = total * COUT, nword = nval / 8;
+  for (int64_t q = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; q < nword; q += int64_t(gridDim.x) * blockDim.x) {
+    const uint4 w = *reinterpret_cast<const uint4 *>(dz + 8 * q);
+    const uint32_t u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-    for (int c = 0; c < COUT; ++c) acc[c] += bf2f(dz[q * COUT + c]);
+    for (int c = 0; c < 4; ++c) {
+      acc[2 * c] += bf2f(uint16_t(u[c] & 0xffff));
+      acc[2 * c + 1] += bf2f(uint16_t(u[c] >> 16));
+    }
+  }
+  if (COUT == 1 && blockIdx.x == 0 && threadIdx.x == 0)
+    for (int64_t q = 8 * nword; q < nval; ++q) acc[0] += bf2f(dz[q]);
+  if (COUT == 1) {
 #pragma unroll
-  for (int c = 0; c < COUT; ++c) {
+    for (int c = 1; c < 8; ++c) acc[0] += acc[c];
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int c = 0; c < (COUT == 1 ? 1 : 8); ++c) {
     float v = acc[c];
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(&db[c], v);
+    for (int off = 32; off >= H; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (lane < H) red[wave][8 * lane + c] = v;  // lane parity: channels 0..7 or 8..15
   }
+  __syncthreads();
+  if (threadIdx.x < COUT)
+    part[int64_t(blockIdx.x) * COUT + threadIdx.x] =
+        (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
 // Adam on the FP32 master parameters
@@ -358,7 +494,7 @@ LpcState::~LpcState() { release(); }
 
 void LpcState::release() {
   for (DevBuf *b : {&wbf, &bias, &vnorm, &x0, &a1, &a2, &y, &dyb, &dz1, &dz2, &sval, &gg, &part, &grad, &master, &mom1,
-                    &mom2, &lsum, &diag, &tbuf})
+                    &mom2, &lsum, &diag, &tbuf, &xq, &dq})
     b->release();
 }
 
@@ -427,13 +563,18 @@ int ensure_acts(rsg_ctx *ctx, int nsamp, bool training) {
 
 template <int CIN, int KP, int MODE, typename T>
 void launch_conv(rsg_ctx *ctx, int nsamp, const uint16_t *in, int64_t in_stride, const uint16_t *w,
-                 const float *bias, uint16_t *out, const uint16_t *mask, float *yout, const T *gsrc, T *pg,
-                 int64_t ldg, const float *sval) {
+                 const float *bias, uint16_t *out, const uint16_t *mask, float *yout, T *pg, int64_t ldg,
+                 const float *sval) {
   const Grid3 g{ctx->n[0], ctx->n[1], ctx->n[2]};
-  const int64_t per = 16 * kTiles * kWaves;
-  dim3 grid(unsigned((ctx->N + per - 1) / per), nsamp);
-  hipLaunchKernelGGL((k_conv<CIN, KP, MODE, T>), grid, dim3(64 * kWaves), 0, ctx->stream, g, ctx->N, in, in_stride,
-                     w, bias, out, mask, yout, gsrc, pg, ldg, sval);
+  const int ntg = (g.n1 * g.n2 + 16 * kWaves - 1) / (16 * kWaves);
+  // whole z-columns where they fill the chip (4 waves a SIMD: 1024 blocks),
+  // else runs of at least four planes (each run reads two planes more)
+  const int64_t cols = int64_t(ntg) * nsamp;
+  int nzr = int(std::min<int64_t>(std::max(1, g.n3 / 4), (2048 + cols - 1) / cols));
+  const int zlen = (g.n3 + nzr - 1) / nzr;
+  nzr = (g.n3 + zlen - 1) / zlen;
+  hipLaunchKernelGGL((k_conv<CIN, KP, MODE, T>), dim3(unsigned(cols * nzr)), dim3(64 * kWaves), 0, ctx->stream, g,
+                     ctx->N, zlen, nzr, ntg, in, in_stride, w, bias, out, mask, yout, pg, ldg, sval);
 }
 
 // forward through all layers for nsamp samples g[smp*ldg + p]; y -> L.y;
@@ -466,28 +607,48 @@ int forward_t(rsg_ctx *ctx, const T *g, int64_t ldg, int nsamp, T *pg, bool trai
   const uint16_t *w1 = L.wbf.as<uint16_t>(), *w2 = w1 + 16 * KP1, *w3 = w2 + 16 * KP2;
   const float *b = L.bias.as<float>();
   launch_conv<2, KP1, kReluOut, T>(ctx, nsamp, L.x0.as<uint16_t>(), N * 2, w1, b, L.a1.as<uint16_t>(), nullptr,
-                                   nullptr, nullptr, nullptr, 0, nullptr);
+                                   nullptr, nullptr, 0, nullptr);
   launch_conv<16, KP2, kReluOut, T>(ctx, nsamp, L.a1.as<uint16_t>(), N * 16, w2, b + 16, L.a2.as<uint16_t>(),
-                                    nullptr, nullptr, nullptr, nullptr, 0, nullptr);
+                                    nullptr, nullptr, nullptr, 0, nullptr);
   launch_conv<16, KP3, kFinalOut, T>(ctx, nsamp, L.a2.as<uint16_t>(), N * 16, w3, b + 32, nullptr, nullptr,
-                                     L.y.as<float>(), g, pg, ldg, L.sval.as<float>());
+                                     L.y.as<float>(), pg, ldg, L.sval.as<float>());
   RSG_HIP(hipGetLastError());
   return RSG_OK;
 }
 
+// quads of a line: one in front, the 16-point chunks, one behind
+int quads_per_line(const rsg_ctx *ctx) { return 4 * ((ctx->n[0] + 15) / 16) + 2; }
+
+template <int C> void to_quads(rsg_ctx *ctx, int nsamp, const uint16_t *in, int wrap, uint16_t *out) {
+  const int64_t nrow = int64_t(ctx->n[1]) * ctx->n[2] * nsamp;
+  const int nq = quads_per_line(ctx);
+  const int64_t n = nrow * nq * C;
+  hipLaunchKernelGGL((k_quads<C>), dim3(unsigned((n + 255) / 256)), dim3(256), 0, ctx->stream, in, nrow, ctx->n[0], nq,
+                     wrap, out);
+}
+
+// gradient of a layer's weights into out and of its biases into db
 template <int CIN, int KP, int COUT>
-int weight_grad(rsg_ctx *ctx, int nsamp, const uint16_t *in, const uint16_t *dz, float *out) {
+int weight_grad(rsg_ctx *ctx, int nsamp, const uint16_t *in, const uint16_t *dz, float *out, float *db) {
   LpcState &L = ctx->lpc;
   const Grid3 g{ctx->n[0], ctx->n[1], ctx->n[2]};
-  const int64_t total = ctx->N * nsamp;
-  const int nblk = int(std::min<int64_t>(512, (total + 4095) / 4096));
-  const int64_t per = (total + nblk - 1) / nblk;
-  if (L.part.ensure(size_t(nblk) * 16 * KP * 4) != hipSuccess) return ctx->fail(RSG_ERR_HIP, "lpc: allocation failed");
-  hipLaunchKernelGGL((k_conv_dw<CIN, KP, COUT>), dim3(nblk), dim3(256), 0, ctx->stream, g, ctx->N, nsamp, in, dz,
-                     per, L.part.as<float>());
+  const int64_t nrow = int64_t(g.n2) * g.n3 * nsamp, total = ctx->N * nsamp;
+  const int nq = quads_per_line(ctx);
+  if (nrow > 0x7fffffff) return ctx->fail(RSG_ERR_UNSUPPORTED, "lpc: too many lines");
+  const int nblk = int(std::min<int64_t>(512, (nrow + 15) / 16));
+  const unsigned nbb = unsigned(std::min<int64_t>(512, (total * COUT + 8 * 256 - 1) / (8 * 256)));
+  if (L.part.ensure(std::max(size_t(nblk) * 16 * KP, size_t(nbb) * COUT) * 4) != hipSuccess ||
+      L.xq.ensure(size_t(nrow) * nq * CIN * 8) != hipSuccess || L.dq.ensure(size_t(nrow) * nq * COUT * 8) != hipSuccess)
+    return ctx->fail(RSG_ERR_HIP, "lpc: allocation failed");
+  float *part = L.part.as<float>();
+  to_quads<CIN>(ctx, nsamp, in, 1, L.xq.as<uint16_t>());
+  to_quads<COUT>(ctx, nsamp, dz, 0, L.dq.as<uint16_t>());
+  hipLaunchKernelGGL((k_conv_dw<CIN, KP, COUT>), dim3(nblk), dim3(256), 0, ctx->stream, g, nsamp, L.xq.as<uint16_t>(),
+                     L.dq.as<uint16_t>(), nq, part);
   const int len = 16 * KP;
-  hipLaunchKernelGGL(k_sum_parts, dim3((len + 255) / 256), dim3(256), 0, ctx->stream, L.part.as<float>(), nblk, len,
-                     out);
+  hipLaunchKernelGGL(k_sum_parts, dim3((len + 63) / 64), dim3(1024), 0, ctx->stream, part, nblk, len, out);
+  hipLaunchKernelGGL(k_bias_grad<COUT>, dim3(nbb), dim3(256), 0, ctx->stream, dz, total, part);
+  hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, ctx->stream, part, int(nbb), COUT, db);
   return RSG_OK;
 }
 
@@ -538,23 +699,17 @@ int lpc_train_step(rsg_ctx *ctx, const float *g, const float *t, int nsamp, floa
                  *w3t = w2t + 16 * KP2;
   // dz2 = (W3' * dy) masked by a2 > 0 ; dz1 = (W2' * dz2) masked by a1 > 0
   launch_conv<1, KP3T, kMaskedGrad, float>(ctx, nsamp, L.dyb.as<uint16_t>(), N, w3t, nullptr, L.dz2.as<uint16_t>(),
-                                           L.a2.as<uint16_t>(), nullptr, nullptr, nullptr, 0, nullptr);
+                                           L.a2.as<uint16_t>(), nullptr, nullptr, 0, nullptr);
   launch_conv<16, KP2, kMaskedGrad, float>(ctx, nsamp, L.dz2.as<uint16_t>(), N * 16, w2t, nullptr,
-                                           L.dz1.as<uint16_t>(), L.a1.as<uint16_t>(), nullptr, nullptr, nullptr, 0,
-                                           nullptr);
+                                           L.dz1.as<uint16_t>(), L.a1.as<uint16_t>(), nullptr, nullptr, 0, nullptr);
   // weight gradients into grad = [G1 16 x KP1 | G2 16 x KP2 | G3 16 x KP3 (row 0)]
-  float *G = L.grad.as<float>();
-  if ((rc = weight_grad<2, KP1, 16>(ctx, nsamp, L.x0.as<uint16_t>(), L.dz1.as<uint16_t>(), G))) return rc;
-  if ((rc = weight_grad<16, KP2, 16>(ctx, nsamp, L.a1.as<uint16_t>(), L.dz2.as<uint16_t>(), G + 16 * KP1))) return rc;
-  if ((rc = weight_grad<16, KP3, 1>(ctx, nsamp, L.a2.as<uint16_t>(), L.dyb.as<uint16_t>(), G + 16 * (KP1 + KP2))))
+  float *G = L.grad.as<float>(), *db = G + 16 * (KP1 + KP2 + KP3);
+  if ((rc = weight_grad<2, KP1, 16>(ctx, nsamp, L.x0.as<uint16_t>(), L.dz1.as<uint16_t>(), G, db))) return rc;
+  if ((rc = weight_grad<16, KP2, 16>(ctx, nsamp, L.a1.as<uint16_t>(), L.dz2.as<uint16_t>(), G + 16 * KP1, db + 16)))
     return rc;
-  float *db = G + 16 * (KP1 + KP2 + KP3);
-  RSG_HIP(hipMemsetAsync(db, 0, 33 * 4, ctx->stream));
-  const int64_t tot = N * nsamp;
-  const unsigned nbb = unsigned(std::min<int64_t>(1024, (tot + 255) / 256));
-  hipLaunchKernelGGL(k_bias_grad<16>, dim3(nbb), dim3(256), 0, ctx->stream, L.dz1.as<uint16_t>(), tot, db);
-  hipLaunchKernelGGL(k_bias_grad<16>, dim3(nbb), dim3(256), 0, ctx->stream, L.dz2.as<uint16_t>(), tot, db + 16);
-  hipLaunchKernelGGL(k_bias_grad<1>, dim3(nbb), dim3(256), 0, ctx->stream, L.dyb.as<uint16_t>(), tot, db + 32);
+  if ((rc = weight_grad<16, KP3, 1>(ctx, nsamp, L.a2.as<uint16_t>(), L.dyb.as<uint16_t>(), G + 16 * (KP1 + KP2),
+                                    db + 32)))
+    return rc;
   RSG_HIP(hipGetLastError());
   // gather into the parameter layout on the host (8241 floats)
   std::vector<float> Gh(size_t(16) * (KP1 + KP2 + KP3) + 33);
