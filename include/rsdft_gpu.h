@@ -134,10 +134,11 @@ int rsg_hpsi_f64_host(rsg_ctx *ctx, const double *psi, double *hpsi,
 
 /* Launch shape of the hpsi kernels for the current grid, per precision
  * (64 or 32): rows per thread ry (1 or 2), tile rows ty, z-planes per
- * workgroup zlen, bands per Infinity-Cache chunk, band tile bt of the
+ * workgroup zlen, bands per chunk, band tile bt of the
  * nonlocal apply (4/8/16/20/32: 16, 32, 64, 80 or 128 bands per matrix-core
  * wave of the analytic form; the table form's scatter takes 4/8/16, and 8
- * for the others).  Zero fields are derived from the grid.  No reference
+ * for the others).  Zero fields (the default) are derived from the grid and
+ * the bands of each call.  No reference
  * counterpart (launch tuning of this implementation). */
 int rsg_set_hpsi_shape(rsg_ctx *ctx, int precision, int ry, int ty, int zlen,
                        int chunk, int bt);
@@ -159,7 +160,7 @@ int rsg_set_hpsi_proj(rsg_ctx *ctx, int precision, int proj);
  * reference counterpart. */
 int rsg_set_hpsi_proj_lds(rsg_ctx *ctx, int precision, int kib);
 int rsg_get_hpsi_proj_lds(rsg_ctx *ctx, int precision, int *kib);
-/* Segment projections (forms 0 and 2) in 1 (default), 2, 4 or 8 pieces
+/* Segment projections (forms 0 and 2) in 1, 2, 4 (default) or 8 pieces
  * per sphere segment, each piece a wave of its own with its own partial
  * sums: shorter waves read the chords that neighbouring spheres share in a
  * plane closer together in time, so the second read finds them in L2 (the
@@ -185,7 +186,8 @@ int rsg_get_analytic_array(rsg_ctx *ctx, int which, void *out, int64_t *count);
 int rsg_get_hpsi_proj(rsg_ctx *ctx, int precision, int *proj);
 /* Grid points along x per stencil thread: 1, or 2 for the pair kernel
  * (FP32 with md = 6, n1 even, tile rows dividing n2; elsewhere the call
- * falls back to 1).  The getter reports what an nb-band call would use.
+ * falls back to 1); until set, 2 where it fits.  The getter reports what an
+ * nb-band call would use.
  * No reference counterpart. */
 int rsg_set_hpsi_xpoints(rsg_ctx *ctx, int precision, int rx);
 int rsg_get_hpsi_xpoints(rsg_ctx *ctx, int precision, int nb, int *rx);

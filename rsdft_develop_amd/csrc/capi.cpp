@@ -477,11 +477,11 @@ int rsg_set_hpsi_shape(rsg_ctx *ctx, int precision, int ry, int ty, int zlen, in
       (bt != 0 && bt != 4 && bt != 8 && bt != 16 && bt != 20 && bt != 32))
     return ctx->fail(RSG_ERR_ARG, "set_hpsi_shape: ry in 0..2, ty/zlen/chunk >= 0, bt in {0,4,8,16,20,32}");
   rsg::HpsiShape &sh = precision == 64 ? ctx->shape64 : ctx->shape32;
-  sh.ry = ry ? ry : 2;
+  sh.ry = ry;
   sh.ty = ty;
   sh.zlen = zlen;
   sh.chunk = chunk;
-  sh.bt = bt ? bt : 8;
+  sh.bt = bt;
   return RSG_OK;
 }
 
@@ -579,7 +579,8 @@ int rsg_set_hpsi_proj_split(rsg_ctx *ctx, int precision, int pieces) {
 int rsg_get_hpsi_proj_split(rsg_ctx *ctx, int precision, int *pieces) {
   if (!ctx || !pieces) return RSG_ERR_ARG;
   if (precision != 64 && precision != 32) return ctx->fail(RSG_ERR_ARG, "get_hpsi_proj_split: precision 64/32");
-  *pieces = (precision == 64 ? ctx->shape64 : ctx->shape32).psplit;
+  const int p = (precision == 64 ? ctx->shape64 : ctx->shape32).psplit;
+  *pieces = p ? p : rsg::kAutoPieces;
   return RSG_OK;
 }
 

@@ -206,15 +206,18 @@ __global__ __launch_bounds__(512) void k_stencil(const T *psi, T *hpsi, int64_t 
         // six independent partial sums (axis, parity of m) instead of one
         // chain of 3 MD + 1 dependent FMAs: the chain's latency, not the
         // issue rate, otherwise bounds the step
-        T sx[2] = {T(0), T(0)}, sy[2] = {T(0), T(0)};
-        T sz[2] = {(cf.c0 + v[sc][r]) * q[r][(u + MD) % R], T(0)};
+        T sx[2] = {T(0), T(0)}, sy[2] = {T(0), T(0)}, sz[2] = {T(0), T(0)};
 #pragma unroll
         for (int m = 0; m < MD; ++m) {
           sx[m & 1] += cf.c[0][m] * (row[xm[m]] + row[xp[m]]);
           sy[m & 1] += cf.c[1][m] * (col[r + MD - 1 - m] + col[r + MD + 1 + m]);
           sz[m & 1] += cf.c[2][m] * (q[r][(u + MD - 1 - m) % R] + q[r][(u + MD + 1 + m) % R]);
         }
+        // the diagonal last: it cancels most of the neighbours' sum (about
+        // 110 psi at h = 0.285 bohr), so no rounding at that size follows
         T acc = ((sx[0] + sx[1]) + (sy[0] + sy[1])) + (sz[0] + sz[1]);
+        acc += cf.c0 * q[r][(u + MD) % R];
+        acc += v[sc][r] * q[r][(u + MD) % R];
         if (ACC) acc += a[sc][r];
         T *dst = own[r] ? o + colofs[r] + zb2 : dst_dead;
         __builtin_nontemporal_store(acc, dst);
@@ -380,9 +383,7 @@ __global__ __launch_bounds__(512) void k_stencil2(const T *psi, T *hpsi, int64_t
       }
       const V c = q[r][(u + MD) % R];
       // per point three independent partial sums (one per axis)
-      T x0 = T(0), x1 = T(0), y0s = T(0), y1s = T(0);
-      T z0 = (cf.c0 + v[sc][r].x) * c.x;
-      T z1 = (cf.c0 + v[sc][r].y) * c.y;
+      T x0 = T(0), x1 = T(0), y0s = T(0), y1s = T(0), z0 = T(0), z1 = T(0);
 #pragma unroll
       for (int m = 0; m < MD; ++m) {
         x0 += cf.c[0][m] * (xw[MD - 1 - m] + xw[MD + 1 + m]);
@@ -393,8 +394,13 @@ __global__ __launch_bounds__(512) void k_stencil2(const T *psi, T *hpsi, int64_t
         z0 += cf.c[2][m] * (lo.x + hi.x);
         z1 += cf.c[2][m] * (lo.y + hi.y);
       }
+      // the diagonal last, as in k_stencil
       T a0 = (x0 + y0s) + z0;
       T a1 = (x1 + y1s) + z1;
+      a0 += cf.c0 * c.x;
+      a1 += cf.c0 * c.y;
+      a0 += v[sc][r].x * c.x;
+      a1 += v[sc][r].y * c.y;
       if (ACC) {
         a0 += a[sc][r].x;
         a1 += a[sc][r].y;
@@ -1036,49 +1042,103 @@ int launch_stencil(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, cons
   }
 }
 
+// Halo elements per thread of the one-point kernel (its template HM is 1, 2 or 4).
+int stencil_halo(int n1, int md, int ry, int ty) {
+  const int th = round64(n1 * (ty / ry));
+  return (2 * md * n1 + th - 1) / th;
+}
+
 // Complete a launch shape: fields left at zero are derived from the grid,
-// the precision and the number of bands of the call.
+// the precision and the number of bands of the call.  Where the lines lie
+// (us per H psi call, analytic projectors):
+// - rows per thread: two share their y-window, but in FP64 with more than
+//   two halo elements per thread the registers no longer hold the prefetch
+//   (108^3, 480 bands: 11740 with two rows, 7060 with one; 72^3, 160 bands,
+//   two halo elements: 604 with two, 660 with one);
+// - FP32 takes the pair kernel where it fits (72^3, 160 bands: 330 against
+//   395; 108^3, 480 bands: 3800 against 4400);
+// - the analytic form runs all bands at once (72^3, 160 bands FP64 in
+//   chunks of 22: 1160, of 80: 709, whole: 618), its partial projections
+//   within 1 GiB;
+// - four pieces per segment (72^3 FP64, whole: 660 with one, 618 with four;
+//   36^3, 20 bands: 52 and 41);
+// - bands per apply wave: the least padding, then the most bands (160
+//   bands: 80 a wave 604, 32 a wave 620);
+// - z-runs for one block per CU (48^3, 40 bands: one or two runs 83-86, six
+//   runs 94; 24^3, 12 bands: one run 34, six 26).
 HpsiShape resolve_shape(const rsg_ctx *ctx, const HpsiShape &in, size_t s, int nb, bool chunked) {
   HpsiShape sh = in;
   const int n1 = ctx->n[0], n2 = ctx->n[1], n3 = ctx->n[2];
-  if (sh.ry < 1 || sh.ry > 2) sh.ry = 2;
+  if (sh.rx == 0) sh.rx = s == sizeof(float) ? 2 : 1;
+  bool auto_ry = sh.ry < 1 || sh.ry > 2;
+  if (auto_ry) sh.ry = 2;
   if (sh.rx == 2) {  // pair kernel: FP32 only; else the one-point kernel
     if (s != sizeof(float)) sh.rx = 1;
     else if (!pair_fits(n1, n2, ctx->md, sh.ry, sh.ty, s)) {
-      sh.ty = pick_ty_pair(n1, n2, ctx->md, sh.ry, s);
-      if (sh.ty == 0) sh.rx = 1;
+      int ty = pick_ty_pair(n1, n2, ctx->md, sh.ry, s);
+      if (ty == 0 && auto_ry) ty = pick_ty_pair(n1, n2, ctx->md, sh.ry = 1, s);
+      if (ty == 0) sh.rx = 1;
+      else sh.ty = ty;
     }
+    if (sh.rx == 1 && auto_ry) sh.ry = 2;
   } else {
     sh.rx = 1;
   }
-  if (sh.rx == 1 && (sh.ty <= 0 || sh.ty % sh.ry || round64(n1 * (sh.ty / sh.ry)) > 512 ||
-      2 * ctx->md * n1 > 4 * round64(n1 * (sh.ty / sh.ry)) ||
-      (2 * size_t(sh.ty + 2 * ctx->md) * n1 + 64) * s > kMaxDynLds)) {
+  auto ty_bad = [&]() {
+    return sh.ty <= 0 || sh.ty % sh.ry || round64(n1 * (sh.ty / sh.ry)) > 512 ||
+           2 * ctx->md * n1 > 4 * round64(n1 * (sh.ty / sh.ry)) ||
+           (2 * size_t(sh.ty + 2 * ctx->md) * n1 + 64) * s > kMaxDynLds;
+  };
+  if (sh.rx == 1 && auto_ry && s == sizeof(double)) {
+    const int ty = ty_bad() ? pick_ty(n1, n2, ctx->md, 2, s) : sh.ty;
+    if (ty == 0 || stencil_halo(n1, ctx->md, 2, ty) > 2) sh.ry = 1;
+  }
+  if (sh.rx == 1 && ty_bad()) {
     sh.ty = pick_ty(n1, n2, ctx->md, sh.ry, s);
     if (sh.ty == 0) {
       sh.ry = 1;
       sh.ty = pick_ty(n1, n2, ctx->md, 1, s);
     }
   }
+  if (sh.psplit != 1 && sh.psplit != 2 && sh.psplit != 4 && sh.psplit != 8) sh.psplit = kAutoPieces;
+  const bool analytic = chunked && ctx->nl_mode != 1 && ctx->have_ana;
   if (sh.chunk <= 0) {
-    // psi + H psi of one chunk within ~128 MB of Infinity Cache
-    const size_t per_band = size_t(ctx->N) * s;
-    sh.chunk = chunked ? int(std::max<size_t>(1, (size_t(64) << 20) / per_band)) : nb;
+    sh.chunk = nb;
+    if (analytic) {
+      const size_t per_band = size_t(std::max(1, ctx->ana64.nseg)) * sh.psplit * 4 * s;
+      sh.chunk = int(std::min<size_t>(size_t(nb), std::max<size_t>(1, (size_t(1) << 30) / per_band)));
+      const int nch = (nb + sh.chunk - 1) / sh.chunk;
+      sh.chunk = (nb + nch - 1) / nch;  // chunks of equal size
+    } else if (chunked) {
+      // table form: psi + H psi of one chunk within ~128 MB of Infinity Cache
+      sh.chunk = int(std::max<size_t>(1, (size_t(64) << 20) / (size_t(ctx->N) * s)));
+    }
   }
   sh.chunk = std::max(1, std::min(sh.chunk, nb));
   if (sh.zlen <= 0) {
     const int tiles = (n2 + sh.ty - 1) / sh.ty;
-    const int64_t want = 3 * 256;
+    const int64_t want = 256;
     int zr = int(std::max<int64_t>(1, (want + int64_t(tiles) * sh.chunk - 1) / (int64_t(tiles) * sh.chunk)));
-    zr = std::min(zr, std::max(1, n3 / 8));
+    zr = std::min(zr, std::max(1, n3 / 4));
     sh.zlen = (n3 + zr - 1) / zr;
   }
   sh.zlen = std::max(1, std::min(sh.zlen, n3));
-  if (sh.bt != 4 && sh.bt != 8 && sh.bt != 16 && sh.bt != 20 && sh.bt != 32) sh.bt = 8;
+  if (sh.bt != 4 && sh.bt != 8 && sh.bt != 16 && sh.bt != 20 && sh.bt != 32) {
+    sh.bt = 8;
+    if (analytic) {
+      int best = 0;
+      for (int bt : {20, 16, 8, 4}) {
+        const int pad = (sh.chunk + 4 * bt - 1) / (4 * bt) * (4 * bt);
+        if (!best || pad < best) {
+          best = pad;
+          sh.bt = bt;
+        }
+      }
+    }
+  }
   if (sh.order != 0 && sh.order != 1) sh.order = 0;
   if (sh.proj < 0 || sh.proj > 2) sh.proj = 0;
   if (sh.plds < 0 || sh.plds > 64) sh.plds = 0;
-  if (sh.psplit != 1 && sh.psplit != 2 && sh.psplit != 4 && sh.psplit != 8) sh.psplit = 1;
   return sh;
 }
 
@@ -1182,7 +1242,9 @@ int launch_hpsi(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, const H
     AnalyticDev<T> &an = ana_of<T>(ctx);
     T *cp = nullptr, *part = nullptr;
     const bool rows = sh.proj == 1 && row_tiles_fit<T>(ctx, an);
-    const int npc = rows ? 1 : sh.psplit;  // partial slots per segment
+    int npc = rows ? 1 : sh.psplit;  // partial slots per segment
+    if (scr && shape_of<T>(ctx).psplit == 0)  // a caller's scratch takes fewer pieces before it refuses a band
+      while (npc > 1 && size_t(4) * (size_t(an.ngroup) + size_t(an.nseg) * npc) * sizeof(T) + 256 > scr->bytes) npc /= 2;
     const int npart = rows ? an.rt_nslot : an.nseg * npc;
     int rc0 = projection_buffers<T>(ctx, scr, size_t(an.ngroup) * 4, size_t(npart) * 4, sh, &cp, &part);
     if (rc0) return rc0;
