@@ -19,8 +19,8 @@
 //     per-point sliced-ELL table, no atomics.
 // Local part:
 //  4. k_stencil: H psi (+)= (c + V) psi + 13-point-per-axis FD Laplacian
-//     (d_kinetic_sol_module.f90:244-292).  A workgroup owns ty full x-rows
-//     of a z-run; each plane is staged in double-buffered LDS with its
+//     (d_kinetic_sol_module.f90:244-292).  A workgroup owns ty x-rows, or
+//     parts of them, of a z-run; each plane is staged in double-buffered LDS with its
 //     +-MD halo rows (periodic in x inside the row, in y by row wrap: the
 //     bcset_3 halo of bc/bcset_3_module.f90:15-151), the z-neighbours stay
 //     in a per-thread register queue, and each thread computes ry rows so
@@ -81,28 +81,38 @@ __device__ inline unsigned xcd_block(unsigned b, unsigned nblk) {
   return x * q + min(x, r) + b / 8;
 }
 
-template <typename T, int MD, int RY, int HM, bool ACC>
+// GX: the rows in parts of xw points.  At 144^3 a workgroup holds only three
+// full rows (512 threads), so 12 halo rows are re-read for every 3: four
+// halo loads a thread and plane, and the kernel waits on them.  A part of
+// 48 x 16 re-reads 0.9 points per point.  144^3, 300 bands FP64: 12.1 ms per
+// H psi call with full rows, 10.8 with parts; 128^3, 240 bands 5.69 and
+// 5.06; 96^3 2.57 and 2.18; 108^3 3.55 and 3.45.
+template <typename T, int MD, int RY, int HM, bool ACC, bool GX>
 __global__ __launch_bounds__(512) void k_stencil(const T *psi, T *hpsi, int64_t ld, const T *vloc,
                                                  StencilCoef<T> cf, int n1, int n2, int n3,
-                                                 int ty, int zlen, T *dead) {
+                                                 int xw, int ty, int zlen, T *dead) {
   constexpr int PF = ring_pf(MD);
   constexpr int R = 2 * MD + 1 + PF;
   static_assert(R % kHS == 0 && R % 2 == 0, "ring length must be a multiple of the rotations");
   extern __shared__ unsigned char smem_raw[];
   T *lds = reinterpret_cast<T *>(smem_raw);
   const int rows = ty + 2 * MD;
-  const int plane = rows * n1;  // one LDS buffer
+  const int LS = GX ? xw + 2 * MD : n1;  // LDS row
+  const int plane = rows * LS;           // one LDS buffer
   const int G = ty / RY;
   const int tid = threadIdx.x, nthr = blockDim.x;
   // idle lanes write a dead slot of their own past both buffers: one slot
   // shared by a whole wave would serialise its 64 writes
   const int dslot = 2 * plane + (tid & 63);
-  const bool active = tid < n1 * G;
-  const int x = active ? tid % n1 : 0;
-  const int g = active ? tid / n1 : 0;
-  // logical block: y-tile fastest, then z-run, then band
+  const bool active = tid < xw * G;
+  const int x = active ? tid % xw : 0;  // in the tile
+  const int g = active ? tid / xw : 0;
+  // logical block: x-tile fastest, then y-tile, z-run, band
+  const int ntile_x = GX ? (n1 + xw - 1) / xw : 1;
   const int ntile_y = (n2 + ty - 1) / ty, nz = (n3 + zlen - 1) / zlen;
-  const unsigned lb = xcd_block(blockIdx.x, gridDim.x);
+  const unsigned lbx = xcd_block(blockIdx.x, gridDim.x);
+  const int x0 = GX ? int(lbx % unsigned(ntile_x)) * xw : 0;
+  const unsigned lb = GX ? lbx / unsigned(ntile_x) : lbx;
   const int by = int(lb % unsigned(ntile_y)), bz = int((lb / unsigned(ntile_y)) % unsigned(nz));
   const int band = int(lb / unsigned(ntile_y * nz));
   const int y0 = by * ty;
@@ -122,28 +132,37 @@ __global__ __launch_bounds__(512) void k_stencil(const T *psi, T *hpsi, int64_t 
 #pragma unroll
   for (int r = 0; r < RY; ++r) {
     const int y = y0 + g * RY + r;
-    own[r] = active && y < n2;
-    colofs[r] = unsigned(x + (y % n2) * n1);  // rows past n2 in the last tile hold wrapped data
-    lown[r] = active ? (MD + g * RY + r) * n1 + x : dslot;
+    own[r] = active && y < n2 && (!GX || x0 + x < n1);
+    // rows and columns past the grid in the last tile hold wrapped data
+    colofs[r] = unsigned((GX ? (x0 + x) % n1 : x) + (y % n2) * n1);
+    lown[r] = active ? (MD + g * RY + r) * LS + (GX ? MD : 0) + x : dslot;
   }
   int xm[MD], xp[MD];
 #pragma unroll
   for (int m = 0; m < MD; ++m) {
-    xm[m] = wrapi(x - m - 1, n1);
-    xp[m] = wrapi(x + m + 1, n1);
+    xm[m] = GX ? MD + x - m - 1 : wrapi(x - m - 1, n1);
+    xp[m] = GX ? MD + x + m + 1 : wrapi(x + m + 1, n1);
   }
   // halo elements this thread stages: LDS offset and in-plane offset
-  const int nhalo = 2 * MD * n1;
+  const int nrow = 2 * MD * xw, nhalo = nrow + (GX ? 2 * MD * ty : 0);
   int hl[HM];
   unsigned hg[HM];
 #pragma unroll
   for (int k = 0; k < HM; ++k) {
     const int idx = tid + k * nthr;
     const int i = idx < nhalo ? idx : 0;
-    const int hr = i / n1, hx = i - hr * n1;
-    const int lrow = hr < MD ? hr : hr + ty;
-    hl[k] = idx < nhalo ? lrow * n1 + hx : dslot;
-    hg[k] = unsigned(hx + wrapi(y0 - MD + lrow, n2) * n1);
+    int lrow, lcol;  // rows above and below the tile, then (GX) the columns beside it
+    if (!GX || i < nrow) {
+      const int hr = i / xw;
+      lrow = hr < MD ? hr : hr + ty;
+      lcol = i - hr * xw + (GX ? MD : 0);
+    } else {
+      const int hr = (i - nrow) / (2 * MD), hc = i - nrow - hr * 2 * MD;
+      lrow = MD + hr;
+      lcol = hc < MD ? hc : hc + xw;
+    }
+    hl[k] = idx < nhalo ? lrow * LS + lcol : dslot;
+    hg[k] = unsigned((GX ? wrapi(x0 - MD + lcol, n1) : lcol) + wrapi(y0 - MD + lrow, n2) * n1);
   }
   T q[RY][R];
 #pragma unroll
@@ -199,10 +218,10 @@ __global__ __launch_bounds__(512) void k_stencil(const T *psi, T *hpsi, int64_t 
       const unsigned zb2 = unsigned(z) * n12;
       T col[RY + 2 * MD];
 #pragma unroll
-      for (int k = 0; k < RY + 2 * MD; ++k) col[k] = buf[(g * RY + k) * n1 + x];
+      for (int k = 0; k < RY + 2 * MD; ++k) col[k] = buf[(g * RY + k) * LS + (GX ? MD : 0) + x];
 #pragma unroll
       for (int r = 0; r < RY; ++r) {
-        const T *row = buf + (MD + g * RY + r) * n1;
+        const T *row = buf + (MD + g * RY + r) * LS;
         // six independent partial sums (axis, parity of m) instead of one
         // chain of 3 MD + 1 dependent FMAs: the chain's latency, not the
         // issue rate, otherwise bounds the step
@@ -875,8 +894,50 @@ template <> HpsiShape &shape_of<double>(rsg_ctx *ctx) { return ctx->shape64; }
 template <> HpsiShape &shape_of<float>(rsg_ctx *ctx) { return ctx->shape32; }
 
 constexpr size_t kMaxDynLds = 64 * 1024;
+constexpr int kCus = 256;      // compute units
+constexpr int kRunStart = 10;  // planes' worth of time a z-run's ring fill takes
 
 inline int round64(int v) { return (v + 63) / 64 * 64; }
+
+// Workgroup of the one-point kernel for ty tile rows: full x-rows while 512
+// threads cover them, else (FP64, two rows a thread) the rows in nx equal
+// parts, whose columns beside the part are halo too.
+struct RowTile {
+  int nx, xw, threads, halo;  // halo elements per plane
+  size_t lds;
+  bool fits;
+};
+RowTile row_tile(int n1, int md, int ry, int ty, size_t s) {
+  RowTile r{1, n1, 0, 0, 0, false};
+  if (ry < 1 || ty < ry || ty % ry || ty / ry > 512 || n1 > 512) return r;
+  const int G = ty / ry;
+  while (r.xw * G > 512) ++r.nx, r.xw = (n1 + r.nx - 1) / r.nx;
+  const bool parts = r.nx > 1;
+  r.threads = round64(r.xw * G);
+  r.halo = 2 * md * (parts ? r.xw + ty : n1);
+  r.lds = (2 * size_t(ty + 2 * md) * (parts ? r.xw + 2 * md : n1) + 64) * s;
+  r.fits = r.lds <= kMaxDynLds &&
+           (parts ? s == sizeof(double) && ry == 2 && r.halo <= 2 * r.threads : r.halo <= 4 * r.threads);
+  return r;
+}
+
+// Tile rows for rows in parts: 16 to 20, with the least padding (8 to 14
+// rows leave more halo, 24 and more make the parts narrow: 144^3, 300 bands
+// 11.8 ms with 12 rows, 10.8 with 16, 11.9 with 24, 13.7 with 32).
+int pick_ty_parts(int n1, int n2, int md, size_t s) {
+  int best_ty = 0;
+  double best = 1e300;
+  for (int ty = 16; ty <= 20; ty += 2) {
+    const RowTile r = row_tile(n1, md, 2, ty, s);
+    if (!r.fits || r.nx == 1) continue;
+    const double cost = double(r.nx) * r.xw / n1 * double((n2 + ty - 1) / ty * ty) / n2;
+    if (cost < best) {
+      best = cost;
+      best_ty = ty;
+    }
+  }
+  return best_ty;
+}
 
 // Tile rows per workgroup for ry rows per thread: balance idle lanes, the
 // partial last tile and the halo rows each plane re-reads.
@@ -961,32 +1022,34 @@ int launch_stencil2_hm(rsg_ctx *ctx, const float *psi, float *hpsi, int64_t ld, 
   return launch_stencil2_t<RY, 4>(ctx, psi, hpsi, ld, nb, sh, accumulate);
 }
 
-template <typename T, int MD, int RY, int HM>
+template <typename T, int MD, int RY, int HM, bool GX = false>
 int launch_stencil_t(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, const HpsiShape &sh,
                      int accumulate) {
   const int n1 = ctx->n[0], n2 = ctx->n[1], n3 = ctx->n[2];
-  const int G = sh.ty / RY;
-  const int threads = round64(n1 * G);
-  const size_t lds = (2 * size_t(sh.ty + 2 * MD) * n1 + 64) * sizeof(T);
-  if (threads > 512 || lds > kMaxDynLds || 2 * MD * n1 > HM * threads)
-    return ctx->fail(RSG_ERR_UNSUPPORTED, "hpsi: stencil tile does not fit");
-  const int64_t nblk = int64_t((n2 + sh.ty - 1) / sh.ty) * ((n3 + sh.zlen - 1) / sh.zlen) * nb;
+  const RowTile rt = row_tile(n1, MD, RY, sh.ty, sizeof(T));
+  if (!rt.fits || rt.halo > HM * rt.threads) return ctx->fail(RSG_ERR_UNSUPPORTED, "hpsi: stencil tile does not fit");
+  const int64_t nblk = int64_t(rt.nx) * ((n2 + sh.ty - 1) / sh.ty) * ((n3 + sh.zlen - 1) / sh.zlen) * nb;
   if (nblk > 0x7fffffff) return ctx->fail(RSG_ERR_UNSUPPORTED, "hpsi: too many stencil workgroups");
   const dim3 grid{unsigned(nblk), 1u, 1u};
   if (accumulate)
-    hipLaunchKernelGGL((k_stencil<T, MD, RY, HM, true>), grid, dim3(threads), lds, ctx->stream, psi, hpsi, ld,
-                       vloc_of<T>(ctx), make_coef<T>(ctx), n1, n2, n3, sh.ty, sh.zlen, ctx->dead.template as<T>());
+    hipLaunchKernelGGL((k_stencil<T, MD, RY, HM, true, GX>), grid, dim3(rt.threads), rt.lds, ctx->stream, psi, hpsi,
+                       ld, vloc_of<T>(ctx), make_coef<T>(ctx), n1, n2, n3, rt.xw, sh.ty, sh.zlen,
+                       ctx->dead.template as<T>());
   else
-    hipLaunchKernelGGL((k_stencil<T, MD, RY, HM, false>), grid, dim3(threads), lds, ctx->stream, psi, hpsi, ld,
-                       vloc_of<T>(ctx), make_coef<T>(ctx), n1, n2, n3, sh.ty, sh.zlen, ctx->dead.template as<T>());
+    hipLaunchKernelGGL((k_stencil<T, MD, RY, HM, false, GX>), grid, dim3(rt.threads), rt.lds, ctx->stream, psi, hpsi,
+                       ld, vloc_of<T>(ctx), make_coef<T>(ctx), n1, n2, n3, rt.xw, sh.ty, sh.zlen,
+                       ctx->dead.template as<T>());
   return RSG_OK;
 }
 
 template <typename T, int MD, int RY>
 int launch_stencil_hm(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, const HpsiShape &sh,
                       int accumulate) {
-  const int threads = round64(ctx->n[0] * (sh.ty / RY));
-  const int need = (2 * MD * ctx->n[0] + threads - 1) / threads;
+  const RowTile rt = row_tile(ctx->n[0], MD, RY, sh.ty, sizeof(T));
+  if (!rt.fits) return ctx->fail(RSG_ERR_UNSUPPORTED, "hpsi: stencil tile does not fit");
+  const int need = (rt.halo + rt.threads - 1) / rt.threads;
+  if constexpr (std::is_same<T, double>::value && RY == 2)
+    if (rt.nx > 1) return launch_stencil_t<T, MD, RY, 2, true>(ctx, psi, hpsi, ld, nb, sh, accumulate);
   if (need <= 1) return launch_stencil_t<T, MD, RY, 1>(ctx, psi, hpsi, ld, nb, sh, accumulate);
   if (need <= 2) return launch_stencil_t<T, MD, RY, 2>(ctx, psi, hpsi, ld, nb, sh, accumulate);
   return launch_stencil_t<T, MD, RY, 4>(ctx, psi, hpsi, ld, nb, sh, accumulate);
@@ -1042,19 +1105,16 @@ int launch_stencil(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, cons
   }
 }
 
-// Halo elements per thread of the one-point kernel (its template HM is 1, 2 or 4).
-int stencil_halo(int n1, int md, int ry, int ty) {
-  const int th = round64(n1 * (ty / ry));
-  return (2 * md * n1 + th - 1) / th;
-}
-
 // Complete a launch shape: fields left at zero are derived from the grid,
 // the precision and the number of bands of the call.  Where the lines lie
 // (us per H psi call, analytic projectors):
 // - rows per thread: two share their y-window, but in FP64 with more than
 //   two halo elements per thread the registers no longer hold the prefetch
-//   (108^3, 480 bands: 11740 with two rows, 7060 with one; 72^3, 160 bands,
-//   two halo elements: 604 with two, 660 with one);
+//   (108^3, 480 bands: 11740 with two full rows, 7060 with one; 72^3, 160
+//   bands, two halo elements: 604 with two, 660 with one); there the rows go
+//   in parts where n1 is even (k_stencil's figures), and full rows stay for
+//   an odd n1, whose parts start misaligned (99^3, 240 bands: 3782 with full
+//   rows, 4001 with parts; 111 x 107 x 101: 4638 and 4762);
 // - FP32 takes the pair kernel where it fits (72^3, 160 bands: 330 against
 //   395; 108^3, 480 bands: 3800 against 4400);
 // - the analytic form runs all bands at once (72^3, 160 bands FP64 in
@@ -1064,8 +1124,12 @@ int stencil_halo(int n1, int md, int ry, int ty) {
 //   36^3, 20 bands: 52 and 41);
 // - bands per apply wave: the least padding, then the most bands (160
 //   bands: 80 a wave 604, 32 a wave 620);
-// - z-runs for one block per CU (48^3, 40 bands: one or two runs 83-86, six
-//   runs 94; 24^3, 12 bands: one run 34, six 26).
+// - z-runs: a run of zlen planes costs zlen + kRunStart planes' time (ring
+//   fill; 40^3, 27 bands: stencil 44, 27, 18 us in runs of 40, 20, 10), and
+//   the blocks go in rounds of as many as the CUs hold at once; the number
+//   of runs with the least rounds x run cost is taken (40^3, 27 bands: 216
+//   blocks 48.5, 270 blocks, so two rounds, 59.0; 24^3, 12 bands: one run
+//   34, six 26).
 HpsiShape resolve_shape(const rsg_ctx *ctx, const HpsiShape &in, size_t s, int nb, bool chunked) {
   HpsiShape sh = in;
   const int n1 = ctx->n[0], n2 = ctx->n[1], n3 = ctx->n[2];
@@ -1084,14 +1148,14 @@ HpsiShape resolve_shape(const rsg_ctx *ctx, const HpsiShape &in, size_t s, int n
   } else {
     sh.rx = 1;
   }
-  auto ty_bad = [&]() {
-    return sh.ty <= 0 || sh.ty % sh.ry || round64(n1 * (sh.ty / sh.ry)) > 512 ||
-           2 * ctx->md * n1 > 4 * round64(n1 * (sh.ty / sh.ry)) ||
-           (2 * size_t(sh.ty + 2 * ctx->md) * n1 + 64) * s > kMaxDynLds;
-  };
+  auto ty_bad = [&]() { return !row_tile(n1, ctx->md, sh.ry, sh.ty, s).fits; };
   if (sh.rx == 1 && auto_ry && s == sizeof(double)) {
     const int ty = ty_bad() ? pick_ty(n1, n2, ctx->md, 2, s) : sh.ty;
-    if (ty == 0 || stencil_halo(n1, ctx->md, 2, ty) > 2) sh.ry = 1;
+    if (ty == 0 || (row_tile(n1, ctx->md, 2, ty, s).halo > 2 * row_tile(n1, ctx->md, 2, ty, s).threads)) {
+      const int part = ty && n1 % 2 == 0 ? pick_ty_parts(n1, n2, ctx->md, s) : 0;
+      if (part) sh.ty = part;
+      else sh.ry = 1;
+    }
   }
   if (sh.rx == 1 && ty_bad()) {
     sh.ty = pick_ty(n1, n2, ctx->md, sh.ry, s);
@@ -1116,11 +1180,27 @@ HpsiShape resolve_shape(const rsg_ctx *ctx, const HpsiShape &in, size_t s, int n
   }
   sh.chunk = std::max(1, std::min(sh.chunk, nb));
   if (sh.zlen <= 0) {
-    const int tiles = (n2 + sh.ty - 1) / sh.ty;
-    const int64_t want = 256;
-    int zr = int(std::max<int64_t>(1, (want + int64_t(tiles) * sh.chunk - 1) / (int64_t(tiles) * sh.chunk)));
-    zr = std::min(zr, std::max(1, n3 / 4));
-    sh.zlen = (n3 + zr - 1) / zr;
+    int tiles = (n2 + sh.ty - 1) / sh.ty, waves, per_cu;
+    if (sh.rx == 2) {
+      waves = round64((n1 / 2) * (sh.ty / sh.ry)) / 64;
+      per_cu = sh.ry == 1 ? 12 : 8;
+    } else {
+      const RowTile rt = row_tile(n1, ctx->md, sh.ry, sh.ty, s);
+      tiles *= rt.nx;
+      waves = std::max(1, rt.threads / 64);
+      per_cu = sh.ry == 1 && rt.halo <= 2 * rt.threads ? 12 : 8;
+    }
+    const int64_t slots = int64_t(kCus) * std::max(1, per_cu / std::max(1, waves)), blocks = int64_t(tiles) * sh.chunk;
+    int64_t best = 0;
+    for (int zr = 1; zr <= std::max(1, n3 / 4); ++zr) {
+      const int zl = (n3 + zr - 1) / zr;
+      const int64_t cost = (blocks * ((n3 + zl - 1) / zl) + slots - 1) / slots * (zl + kRunStart);
+      if (!best || cost < best) {
+        best = cost;
+        sh.zlen = zl;
+      }
+      if (blocks * zr >= 8 * slots) break;
+    }
   }
   sh.zlen = std::max(1, std::min(sh.zlen, n3));
   if (sh.bt != 4 && sh.bt != 8 && sh.bt != 16 && sh.bt != 20 && sh.bt != 32) {

@@ -204,6 +204,29 @@ def test_pair_stencil_falls_back_where_it_does_not_apply(orc, gpu_mod):
     _f32_local_and_full(ham, ctx, systems.random_bands(cell.npoints, 3, seed=4), cell.npoints + 37)
 
 
+@pytest.mark.parametrize("ngrid,ty,zlen", [((52, 24, 14), 20, 0), ((54, 27, 13), 20, 5), ((72, 35, 15), 18, 4),
+                                           ((57, 20, 16), 18, 0), ((128, 16, 13), 16, 0), ((108, 19, 14), 0, 0)])
+def test_stencil_rows_in_parts(orc, gpu_mod, ngrid, ty, zlen):
+    """Grid rows split over workgroups: parts that do not divide the row,
+    ragged last rows and z-runs, odd rows, and the default's own choice at
+    108 points; against the oracle, and to the last bit against full rows
+    (the same sums in the same order)."""
+    base = systems.silicon_supercell(1, displacement=0.1, seed=5)
+    cell = systems.Cell(aa=np.diag([0.3 * n for n in ngrid]), frac=base.frac, kind=base.kind, species=base.species,
+                        ngrid=ngrid, nband=3, md=6)
+    ham, ctx = _pair(orc, gpu_mod, cell)
+    psi = systems.random_bands(cell.npoints, 3, seed=ngrid[0])
+    ctx.set_hpsi_shape(64, ry=1)
+    full = ctx.hamiltonian(psi)
+    ctx.set_hpsi_shape(64, ry=2 if ty else 0, ty=ty, zlen=zlen)
+    sh = ctx.hpsi_shape(64, 3)
+    print(f"case: rows in parts {ngrid}, shape {sh}", flush=True)
+    assert sh["ry"] == 2 and ngrid[0] * (sh["ty"] // 2) > 512 and (not ty or sh["ty"] == ty)
+    got = ctx.hamiltonian(psi)
+    _close(got, ham.hpsi(psi), 1e-12)
+    np.testing.assert_array_equal(got, full)
+
+
 def test_hpsi_errors(gpu_mod):
     ctx = gpu_mod.Context()
     a = np.zeros((8, 1), order="F")
