@@ -111,61 +111,126 @@ __global__ __launch_bounds__(kThreads) void k_multidot(DotArgs<W> a, int64_t N, 
   }
 }
 
-// out[t] = alpha * sum_s partial[t nseg + s].  Eight lanes per sum: one
-// thread per sum walks nseg dependent loads (5.6 us for 20 sums of 64, a
-// fifth of a small cell's CG call); a fixed order either way.
-constexpr int kRedLanes = 8;
+// out[t] = alpha * sum_s partial[t nseg + s].  Eight lanes per sum, a wave
+// above 64 partials: one thread per sum walks nseg dependent loads (5.6 us
+// for 20 sums of 64, a fifth of a small cell's CG call); a fixed order
+// either way.
+template <int L>
 __global__ void k_reduce_partials(const double *__restrict__ partial, int nseg, int count,
                                   double alpha, double *__restrict__ out) {
-  const int t = (blockIdx.x * blockDim.x + threadIdx.x) / kRedLanes, l = threadIdx.x % kRedLanes;
+  const int t = (blockIdx.x * blockDim.x + threadIdx.x) / L, l = threadIdx.x % L;
   double v = 0.0;
   if (t < count)
-    for (int s = l; s < nseg; s += kRedLanes) v += partial[int64_t(t) * nseg + s];
+    for (int s = l; s < nseg; s += L) v += partial[int64_t(t) * nseg + s];
 #pragma unroll
-  for (int o = kRedLanes / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, kRedLanes);
+  for (int o = L / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, L);
   if (t < count && l == 0) out[t] = alpha * v;
 }
 
 void reduce_partials(rsg_ctx *ctx, const double *partial, int nseg, int count, double alpha, double *out) {
-  constexpr int per = 256 / kRedLanes;
-  hipLaunchKernelGGL(k_reduce_partials, dim3((count + per - 1) / per), dim3(256), 0, ctx->stream, partial, nseg, count,
-                     alpha, out);
+  if (nseg > 64)
+    hipLaunchKernelGGL((k_reduce_partials<64>), dim3((count + 3) / 4), dim3(256), 0, ctx->stream, partial, nseg, count,
+                       alpha, out);
+  else
+    hipLaunchKernelGGL((k_reduce_partials<8>), dim3((count + 31) / 32), dim3(256), 0, ctx->stream, partial, nseg, count,
+                       alpha, out);
 }
 
 // --------------------------------------------------------- band-wise updates
+// The kernels that write the gradient also sum <g, g>: one partial per
+// block of kSeg points (b nseg + s), which saves a read of g and a launch
+// per CG step.  Four points a thread: with long segments instead the reads
+// and writes of all bands advance in step and the update of 480 bands of
+// 108^3 FP64 takes 6.9 ms, so 5.6 (and 6.4 before: one point a thread 5.2,
+// the dot 1.2).  The block's sum, from thread 0:
+constexpr int kSegPts = 4, kSeg = kSegPts * kThreads;
+__device__ inline void seg_partial(double v, double *__restrict__ partial) {
+  __shared__ double red[kThreads / 64];
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    v = 0.0;
+#pragma unroll
+    for (int k = 0; k < kThreads / 64; ++k) v += red[k];
+    partial[int64_t(blockIdx.y) * gridDim.x + blockIdx.x] = v;
+  }
+}
+
 // gk = -2 (hx - E x)          (cg_module.f90:207)
 template <typename W>
-__global__ void k_cg_grad(const W *__restrict__ hx, const W *__restrict__ x, const double *__restrict__ E,
-                          W *__restrict__ g, int64_t N) {
+__global__ __launch_bounds__(kThreads) void k_cg_grad(const W *__restrict__ hx, const W *__restrict__ x,
+                                                      const double *__restrict__ E, W *__restrict__ g, int64_t N,
+                                                      double *__restrict__ partial) {
   const int b = blockIdx.y;
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  const int64_t k = int64_t(b) * N + i;
+  const int64_t i0 = int64_t(blockIdx.x) * kSeg + threadIdx.x, off = int64_t(b) * N;
   const W e = W(E[b]);
-  g[k] = W(-2) * (hx[k] - e * x[k]);
+  double acc = 0.0;
+#pragma unroll
+  for (int u = 0; u < kSegPts; ++u) {
+    const int64_t i = i0 + u * kThreads, k = off + i;
+    if (i >= N) break;
+    const W v = W(-2) * (hx[k] - e * x[k]);
+    g[k] = v;
+    acc += double(v) * double(v);
+  }
+  seg_partial(acc, partial);
 }
 
 // y = x (first step) or y = x + (rb/gkgk) y   (cg_module.f90:266-279);
 // a zero previous <Pg, g> (a band whose gradient vanished) restarts the
-// direction instead of forming 0/0
-template <typename W>
+// direction instead of forming 0/0.  With XM != 0 the step before this one
+// is accepted on the way, as k_cg_accept (XM 1, FP64 store) and
+// k_cg_accept32 (XM 2) do: its direction is read here anyway (480 bands of
+// 108^3 FP64: 4.2 ms a step, direction and acceptance apart 4.7).
+template <typename W, int XM>
 __global__ void k_cg_dir(const W *__restrict__ pg, W *__restrict__ pk, const double *__restrict__ rb,
-                         const double *__restrict__ gkgk, int first, int64_t N) {
+                         const double *__restrict__ gkgk, int first, int64_t N, double *__restrict__ x,
+                         W *__restrict__ xw, const double *__restrict__ uc, const int *__restrict__ accept) {
   const int b = blockIdx.y;
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= N) return;
   const int64_t k = int64_t(b) * N + i;
   const double bk = gkgk[b] != 0.0 ? rb[b] / gkgk[b] : 0.0;
-  pk[k] = first ? pg[k] : pg[k] + W(bk) * pk[k];
+  if (first) {
+    pk[k] = pg[k];
+    return;
+  }
+  const W p = pk[k];
+  pk[k] = pg[k] + W(bk) * p;
+  if (XM && accept[b]) {
+    if (XM == 1) {
+      const double v = uc[2 * b] * x[k] + uc[2 * b + 1] * double(p);
+      x[k] = v;
+      if (xw) xw[k] = W(v);
+    } else {
+      xw[k] = W(uc[2 * b] * double(xw[k]) + uc[2 * b + 1] * double(p));
+    }
+  }
 }
 
 // 2x2 generalised Ritz step per band (cg_module.f90:305-334): DSYGV on
-// (<x,p|H|x,p>, <x,p|x,p>), root switch, sign fix.  d6 holds
-// (xx, px, pp, xHx, pHx, pHp) * dV as [q*nb + b].
-__global__ void k_cg_ritz(const double *__restrict__ d6, int nb, double *__restrict__ E,
-                          double *__restrict__ E1, double *__restrict__ uc, const int *__restrict__ done) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nb) return;
+// (<x,p|H|x,p>, <x,p|x,p>), root switch, sign fix.  One wave per band
+// finishes the sums of k_ritz_dots, (xx, px, pp, xHx, pHx, pHp), times dV;
+// the step's <Pg, g> becomes the previous one.
+__global__ __launch_bounds__(kThreads) void k_cg_ritz(const double *__restrict__ partial, int nseg, double dv, int nb,
+                                                      double *__restrict__ E, double *__restrict__ E1,
+                                                      double *__restrict__ uc, const double *__restrict__ rb,
+                                                      double *__restrict__ gkgk, const int *__restrict__ done) {
+  const int b = (blockIdx.x * blockDim.x + threadIdx.x) / 64, lane = threadIdx.x & 63;
+  if (b >= nb) return;  // whole waves
+  double d6[6];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    double v = 0.0;
+    for (int s = lane; s < nseg; s += 64) v += partial[(int64_t(q) * nb + b) * nseg + s];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+    d6[q] = dv * v;
+  }
+  if (lane) return;
+  gkgk[b] = rb[b];
   if (*done) {
     // the block has converged (the reference leaves the CG loop here): the
     // remaining steps keep every band, u = (1, 0), E unchanged
@@ -174,8 +239,8 @@ __global__ void k_cg_ritz(const double *__restrict__ d6, int nb, double *__restr
     E1[b] = E[b];
     return;
   }
-  const double b11 = d6[0 * nb + b], b12 = d6[1 * nb + b], b22 = d6[2 * nb + b];
-  const double a11 = d6[3 * nb + b], a12 = d6[4 * nb + b], a22 = d6[5 * nb + b];
+  const double b11 = d6[0], b12 = d6[1], b22 = d6[2];
+  const double a11 = d6[3], a12 = d6[4], a22 = d6[5];
   // B = U^T U, C = U^-T A U^-1, C = Y diag(w) Y^T, X = U^-1 Y
   const double u11 = sqrt(b11), u12 = b12 / u11, u22 = sqrt(b22 - u12 * u12);
   const double i11 = 1.0 / u11, i12 = -u12 / (u11 * u22), i22 = 1.0 / u22;
@@ -226,31 +291,73 @@ __global__ void k_cg_ritz(const double *__restrict__ d6, int nb, double *__restr
 
 // hx <- u1 hx + u2 hp ; g <- -2 (hx - W (u1 x + u2 p))   (cg_module.f90:336-352)
 template <typename W>
-__global__ void k_cg_update(W *__restrict__ hx, const W *__restrict__ hp, const W *__restrict__ x,
-                            const W *__restrict__ p, W *__restrict__ g, const double *__restrict__ uc,
-                            const double *__restrict__ E, int64_t N) {
+__global__ __launch_bounds__(kThreads) void k_cg_update(W *__restrict__ hx, const W *__restrict__ hp,
+                                                        const W *__restrict__ x, const W *__restrict__ p,
+                                                        W *__restrict__ g, const double *__restrict__ uc,
+                                                        const double *__restrict__ E, int64_t N,
+                                                        double *__restrict__ partial) {
   const int b = blockIdx.y;
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  const int64_t k = int64_t(b) * N + i;
+  const int64_t i0 = int64_t(blockIdx.x) * kSeg + threadIdx.x, off = int64_t(b) * N;
   const W u1 = W(uc[2 * b]), u2 = W(uc[2 * b + 1]), ev = W(E[b]);
-  const W h = u1 * hx[k] + u2 * hp[k];
-  hx[k] = h;
-  g[k] = W(-2) * (h - ev * (u1 * x[k] + u2 * p[k]));
+  double acc = 0.0;
+#pragma unroll
+  for (int u = 0; u < kSegPts; ++u) {
+    const int64_t i = i0 + u * kThreads, k = off + i;
+    if (i >= N) break;
+    const W h = u1 * hx[k] + u2 * hp[k];
+    hx[k] = h;
+    const W v = W(-2) * (h - ev * (u1 * x[k] + u2 * p[k]));
+    g[k] = v;
+    acc += double(v) * double(v);
+  }
+  seg_partial(acc, partial);
 }
 
-// divergence guard (cg_module.f90:358-364): reject when rb/res > 1e8, and
-// also when the new gradient norm is not finite (the reference would carry
-// a NaN into the band); an exactly zero gradient before and after (0/0)
-// keeps the band, which the Ritz step left unchanged
-__global__ void k_cg_guard(const double *__restrict__ rb, const double *__restrict__ res,
-                           double *__restrict__ E, const double *__restrict__ E1,
-                           int *__restrict__ accept, int nb) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nb) return;
-  const int ok = std::isfinite(rb[b]) && !(rb[b] / res[b] > 1.0e8);
-  accept[b] = ok;
-  if (!ok) E[b] = E1[b];
+// One block ends a CG step: rb = dV <g, g> from the gradient's partials,
+// 16 lanes per band, then
+// - the divergence guard (cg_module.f90:358-364): reject when rb/res > 1e8,
+//   and also when the new gradient norm is not finite (the reference would
+//   carry a NaN into the band); an exactly zero gradient before and after
+//   (0/0) keeps the band, which the Ritz step left unchanged;
+// - res = rb / 4 (:231);
+// - the convergence test (:236), |E - E1| < 1e-15 for the whole block,
+//   sticky for the rest of the call: the remaining steps leave the block as
+//   it is (the reference exits the loop), without a read-back per step.
+// first: the gradient before the first step, rb and res only.
+constexpr int kGuardThreads = 1024;
+__global__ __launch_bounds__(kGuardThreads) void k_cg_guard(const double *__restrict__ partial, int nseg, double dv,
+                                                            int first, double *__restrict__ rb,
+                                                            double *__restrict__ res, double *__restrict__ E,
+                                                            const double *__restrict__ E1, int *__restrict__ accept,
+                                                            int nb, int *__restrict__ flag) {
+  constexpr int L = 16, PER = kGuardThreads / L;
+  __shared__ int any_moving;
+  if (threadIdx.x == 0) any_moving = 0;
+  __syncthreads();
+  const int l = threadIdx.x % L;
+  int moving = 0;
+  for (int b0 = 0; b0 < nb; b0 += PER) {
+    const int b = b0 + threadIdx.x / L;
+    double v = 0.0;
+    if (b < nb)
+      for (int s = l; s < nseg; s += L) v += partial[int64_t(b) * nseg + s];
+#pragma unroll
+    for (int o = L / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, L);
+    if (b >= nb || l) continue;
+    const double r = dv * v;
+    rb[b] = r;
+    if (!first) {
+      const int ok = std::isfinite(r) && !(r / res[b] > 1.0e8);
+      accept[b] = ok;
+      if (!ok) E[b] = E1[b];
+      moving |= !(fabs(E[b] - E1[b]) < 1e-15);
+    }
+    res[b] = 0.25 * r;
+  }
+  if (first) return;
+  if (moving) atomicOr(&any_moving, 1);
+  __syncthreads();
+  if (threadIdx.x == 0 && !any_moving) *flag = 1;
 }
 
 // x <- u1 x + u2 p for accepted bands (cg_module.f90:366)
@@ -388,20 +495,6 @@ __global__ void k_all_below(const double *__restrict__ v, int nb, double bound, 
   if (above) atomicOr(&any_above, 1);
   __syncthreads();
   if (threadIdx.x == 0) *flag = any_above ? 0 : 1;
-}
-
-// flag |= all(|E - E1| < 1e-15): the CG block's convergence test
-// (cg_module.f90:236), sticky for the rest of the call
-__global__ void k_cg_conv(const double *__restrict__ E, const double *__restrict__ E1, int nb,
-                          int *__restrict__ flag) {
-  __shared__ int any_moving;
-  if (threadIdx.x == 0) any_moving = 0;
-  __syncthreads();
-  int moving = 0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) moving |= !(fabs(E[b] - E1[b]) < 1e-15);
-  if (moving) atomicOr(&any_moving, 1);
-  __syncthreads();
-  if (threadIdx.x == 0 && !any_moving) *flag = 1;
 }
 
 __global__ void k_fill_int(int *__restrict__ a, int v, int n) {
@@ -1122,7 +1215,7 @@ inline dim3 grid_nb(int64_t N, int nb) { return dim3(unsigned((N + kThreads - 1)
 
 struct Scratch {
   // per-band device scalars, each nb doubles
-  double *E, *E1, *rb, *gkgk, *res, *d6, *uc, *rr0, *rr1, *a, *pap;
+  double *E, *E1, *rb, *gkgk, *res, *uc, *rr0, *rr1, *a, *pap;
   int *accept;
   // device-side decisions: flags[0] the CG block has converged, flags[1]
   // the preconditioner's first residuals are all below its exit bound
@@ -1132,7 +1225,7 @@ struct Scratch {
 int ensure_scalars(rsg_ctx *ctx, int nb, int nseg, Scratch &s) {
   const size_t per = size_t(nb);
   (void)nseg;
-  const size_t nd = per * (9 + 6 + 2);
+  const size_t nd = per * (9 + 2);
   if (ctx->scal.ensure(nd * sizeof(double) + per * sizeof(int) + 256) != hipSuccess)
     return ctx->fail(RSG_ERR_HIP, "solver: scalar scratch allocation failed");
   double *p = ctx->scal.as<double>();
@@ -1145,18 +1238,20 @@ int ensure_scalars(rsg_ctx *ctx, int nb, int nseg, Scratch &s) {
   s.rr1 = p; p += per;
   s.a = p; p += per;
   s.pap = p; p += per;
-  s.d6 = p; p += 6 * per;
   s.uc = p; p += 2 * per;
   s.accept = reinterpret_cast<int *>(p);
   s.flags = s.accept + per;  // 4 ints inside the 256-byte tail
   return RSG_OK;
 }
 
+// Segments of a dot product: enough blocks to fill the chip (8 four-wave
+// blocks per CU, twice), each of 1024 points or more (36^3, 20 bands: the
+// Ritz products 14.1 us in segments of 4096 and up, 8.5 in 1024 and up; 512
+// gives no more).
+constexpr int64_t kSegBlocks = 4096, kSegMin = 1024;
 int seg_count(int64_t N, int nb) {
   int nseg = 1;
-  // enough blocks to fill the chip (8 four-wave blocks per CU), each
-  // segment at least 4096 points
-  while (nseg < 64 && int64_t(nseg) * nb < 4096 && N / (nseg * 2) >= 4096) nseg *= 2;
+  while (nseg < 64 && int64_t(nseg) * nb < kSegBlocks && N / (nseg * 2) >= kSegMin) nseg *= 2;
   return nseg;
 }
 
@@ -1208,20 +1303,15 @@ int multidot(rsg_ctx *ctx, int npair, const double *const *x, const double *cons
 
 namespace {
 
-// out[q*nb + b] = alpha * the six Ritz-step products of band b
+// partial sums of the six Ritz-step products, for k_cg_ritz
 template <typename W>
-int ritz_dots(rsg_ctx *ctx, const W *x, const W *p, const W *hx, const W *hp, int nb, double alpha, double *out) {
-  if (nb == 0) return RSG_OK;
+int ritz_dots(rsg_ctx *ctx, const W *x, const W *p, const W *hx, const W *hp, int nb) {
   const int64_t N = ctx->N;
   const int nseg = seg_count(N, nb);
-  const int64_t seglen = (N + nseg - 1) / nseg;
   if (ctx->dotpart.ensure(size_t(6) * nb * nseg * sizeof(double)) != hipSuccess)
     return ctx->fail(RSG_ERR_HIP, "ritz_dots: scratch allocation failed");
-  double *partial = ctx->dotpart.as<double>();
   hipLaunchKernelGGL((k_ritz_dots<W>), dim3(nseg, nb), dim3(kThreads), 0, ctx->stream, x, p, hx, hp, N, nb, nseg,
-                     seglen, partial);
-  const int count = 6 * nb;
-  reduce_partials(ctx, partial, nseg, count, alpha, out);
+                     (N + nseg - 1) / nseg, ctx->dotpart.as<double>());
   return RSG_OK;
 }
 
@@ -2053,18 +2143,27 @@ int cg_impl(rsg_ctx *ctx, int ncg, int pc_kind, int mloop, double *esp, double *
       const W *xs[1] = {x}, *ys[1] = {hxk};
       if ((rc = multidot(ctx, 1, xs, ys, nn, dv, s.E))) return rc;
     }
-    hipLaunchKernelGGL((k_cg_grad<W>), gN, blkd, 0, ctx->stream, hxk, x, s.E, gk, N);
-    {
-      const W *xs[1] = {gk}, *ys[1] = {gk};
-      if ((rc = multidot(ctx, 1, xs, ys, nn, dv, s.rb))) return rc;
-    }
-    for (int icg = 1; icg <= ncg + 1; ++icg) {
-      hipLaunchKernelGGL(k_scale_copy, gb, b64, 0, ctx->stream, s.rb, 0.25, s.res, nn);
-      if (icg == ncg + 1) break;
-      // convergence test on the device: once the whole block has
-      // |E - E1| < 1e-15 the remaining steps leave it as it is (the
-      // reference exits the loop), without a read-back per step
-      hipLaunchKernelGGL(k_cg_conv, dim3(1), dim3(256), 0, ctx->stream, s.E, s.E1, nn, s.flags);
+    const int nseg = seg_count(N, nn);
+    const int ngg = int((N + kSeg - 1) / kSeg);  // partials of <g, g>
+    if (ctx->dotpart.ensure((size_t(ngg) + 1) * nn * sizeof(double)) != hipSuccess)
+      return ctx->fail(RSG_ERR_HIP, "conjugate_gradient: scratch allocation failed");
+    const dim3 gS(ngg, nn);
+    auto part = [&]() { return ctx->dotpart.as<double>(); };  // the preconditioner may grow it
+    auto end_step = [&](int first) {
+      const double *pt = part();
+      if (ngg > 64) {  // too many for the guard's one block
+        reduce_partials(ctx, pt, ngg, nn, 1.0, part() + size_t(ngg) * nn);
+        pt += size_t(ngg) * nn;
+      }
+      hipLaunchKernelGGL(k_cg_guard, dim3(1), dim3(kGuardThreads), 0, ctx->stream, pt, ngg > 64 ? 1 : ngg, dv, first, s.rb, s.res,
+                         s.E, s.E1, s.accept, nn, s.flags);
+    };
+    hipLaunchKernelGGL((k_cg_grad<W>), gS, blkd, 0, ctx->stream, hxk, x, s.E, gk, N, part());
+    end_step(1);
+    // a step's bands are accepted with the next direction; at once after
+    // the last one, and where the next step's projection reads the store
+    const bool defer = ctx->cg_swgs == 0;
+    for (int icg = 1; icg <= ncg; ++icg) {
       // pgk = P gk and rb = dV <pgk, gk>; once the network's output has
       // failed the descent check in this call, the block keeps the hprsdft
       // smoother for the rest of the call
@@ -2118,18 +2217,24 @@ int cg_impl(rsg_ctx *ctx, int ncg, int pc_kind, int mloop, double *esp, double *
         const W *xs[1] = {pgk}, *ys[1] = {gk};
         if ((rc = multidot(ctx, 1, xs, ys, nn, dv, s.rb))) return rc;
       }
-      hipLaunchKernelGGL((k_cg_dir<W>), gN, blkd, 0, ctx->stream, pgk, pk, s.rb, s.gkgk, icg == 1 ? 1 : 0, N);
-      hipLaunchKernelGGL(k_scale_copy, gb, b64, 0, ctx->stream, s.rb, 1.0, s.gkgk, nn);
+      if (icg == 1 || !defer)
+        hipLaunchKernelGGL((k_cg_dir<W, 0>), gN, blkd, 0, ctx->stream, pgk, pk, s.rb, s.gkgk, icg == 1 ? 1 : 0, N,
+                           nullptr, nullptr, s.uc, s.accept);
+      else if (in_place)
+        hipLaunchKernelGGL((k_cg_dir<W, 2>), gN, blkd, 0, ctx->stream, pgk, pk, s.rb, s.gkgk, 0, N, nullptr, x, s.uc,
+                           s.accept);
+      else
+        hipLaunchKernelGGL((k_cg_dir<W, 1>), gN, blkd, 0, ctx->stream, pgk, pk, s.rb, s.gkgk, 0, N, xs64, x32, s.uc,
+                           s.accept);
       if ((rc = launch_hpsi<W>(ctx, pk, hpk, N, nn))) return rc;
-      if ((rc = ritz_dots<W>(ctx, x, pk, hxk, hpk, nn, dv, s.d6))) return rc;
-      hipLaunchKernelGGL(k_cg_ritz, gb, b64, 0, ctx->stream, s.d6, nn, s.E, s.E1, s.uc, s.flags);
-      hipLaunchKernelGGL((k_cg_update<W>), gN, blkd, 0, ctx->stream, hxk, hpk, x, pk, gk, s.uc, s.E, N);
-      {
-        const W *xs[1] = {gk}, *ys[1] = {gk};
-        if ((rc = multidot(ctx, 1, xs, ys, nn, dv, s.rb))) return rc;
-      }
-      hipLaunchKernelGGL(k_cg_guard, gb, b64, 0, ctx->stream, s.rb, s.res, s.E, s.E1, s.accept, nn);
-      if (in_place)
+      if ((rc = ritz_dots<W>(ctx, x, pk, hxk, hpk, nn))) return rc;
+      hipLaunchKernelGGL(k_cg_ritz, dim3((nn + 3) / 4), dim3(kThreads), 0, ctx->stream, part(), nseg, dv, nn, s.E, s.E1,
+                         s.uc, s.rb, s.gkgk, s.flags);
+      hipLaunchKernelGGL((k_cg_update<W>), gS, blkd, 0, ctx->stream, hxk, hpk, x, pk, gk, s.uc, s.E, N, part());
+      end_step(0);
+      if (defer && icg < ncg) {
+        // with the next direction
+      } else if (in_place)
         hipLaunchKernelGGL((k_cg_accept32<W>), gN, blkd, 0, ctx->stream, x, pk, s.uc, s.accept, N);
       else
         hipLaunchKernelGGL((k_cg_accept<W>), gN, blkd, 0, ctx->stream, xs64, x32, pk, s.uc, s.accept, N);

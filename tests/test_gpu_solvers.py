@@ -572,3 +572,28 @@ def test_precond_hprsdft_near_eigenvectors(orc, ngrid, mloop):
             continue
         err = np.abs(got[:, b] - want[:, b]).max() / np.abs(want[:, b]).max()
         assert err <= 1e-12, (b, err)
+
+
+@pytest.mark.parametrize("ngrid", [(16, 8, 8), (31, 13, 11), (42, 42, 42)])
+@pytest.mark.parametrize("ncg", [0, 1, 3])
+def test_conjugate_gradient_step_counts_and_grid_sizes(orc, ngrid, ncg):
+    """Bands accepted with the next direction or, after the last step, at
+    once, and the gradient's norm summed with its update: one whole block of
+    points, a remainder, and more blocks than the step's last kernel sums
+    itself.  Tolerances as of the Si8 comparison: summation order only."""
+    from rsdft_develop_amd import gpu
+
+    base = systems.silicon_supercell(1, displacement=0.05, seed=4)
+    cell = systems.Cell(aa=np.diag([0.3 * n for n in ngrid]), frac=base.frac, kind=base.kind, species=base.species,
+                        ngrid=ngrid, nband=3, md=6)
+    v = systems.model_vloc(cell)
+    ham = orc.Ham(cell, vloc=v)
+    ctx = gpu.Context().setup(cell, v)
+    u, _ = ham.subspace_diag(ham.gram_schmidt(systems.random_bands(cell.npoints, 3, seed=6), "lusl"))
+    _load(ctx, u)
+    print(f"case: CG {ngrid}, {ncg} steps", flush=True)
+    esp, res = ctx.conjugate_gradient(ncg=ncg, pc_kind=4, mloop=3)
+    u_want, esp_want, res_want = ham.conjugate_gradient(u, ncg=ncg, pc_kind=4)
+    np.testing.assert_allclose(esp, esp_want, atol=1e-9)
+    np.testing.assert_allclose(res, res_want, rtol=1e-7, atol=1e-12)
+    assert np.abs(ctx.download_bands() - u_want).max() < 1e-7 * np.abs(u_want).max()
