@@ -1611,56 +1611,210 @@ int precond_hprsdft_fused(rsg_ctx *ctx, int mloop, const W *g, W *pg, int nn, W 
 }  // namespace
 
 namespace {
-// out[t] = alpha * sum_c part[c * count + t]
-__global__ void k_sum_batches(const double *__restrict__ part, int nbat, int count, double alpha,
-                              double *__restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= count) return;
-  double v = 0.0;
-  for (int c = 0; c < nbat; ++c) v += part[int64_t(c) * count + t];
-  out[t] = alpha * v;
+// C (nb x nb) = A^T B with A, B column-major N x nb: K = N is long and the
+// output a few tiles, so the points are split over blocks too.  A block
+// takes a square tile of 16 TI bands a side and kc points; its four waves
+// take a quarter of the points each, straight from memory into matrix-core
+// operands (which point goes to which k of the product is free as long as A
+// and B agree: a lane holds four consecutive points, so 16 bands x 128
+// bytes a load), and add their tiles through LDS.  Tiles run fastest in the
+// block order and every XCD walks one contiguous range of points, so a band
+// comes from HBM about once and from that XCD's L2 for the other tiles.
+// SYM (A = B): tiles of the upper triangle only.
+template <int TI, bool SYM>
+__global__ __launch_bounds__(256, TI == 3 ? 2 : 3) void k_gram(const double *__restrict__ A, const double *__restrict__ B, int64_t N,
+                                              int nb, int64_t kc, int nt, int ntile, double *__restrict__ part) {
+  typedef double V4 __attribute__((ext_vector_type(4)));
+  typedef double U4 __attribute__((ext_vector_type(4), aligned(8)));  // bands start at odd multiples of 8 bytes for odd N
+  constexpr int T = 16 * TI;
+  const int tid = threadIdx.x, l = tid & 63, lo = l & 15, hi = l >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const unsigned nblk = gridDim.x, xc = blockIdx.x % 8;
+  const unsigned lb = xc * (nblk / 8) + min(xc, nblk % 8) + blockIdx.x / 8;
+  const int tile = int(lb % unsigned(ntile));
+  const int64_t chunk = lb / unsigned(ntile);
+  int ti, tj;
+  if (SYM) {  // column tj holds tiles 0 .. tj
+    tj = 0;
+    for (int s = tile; s > tj; s -= tj) ++tj;
+    ti = tile - tj * (tj + 1) / 2;
+  } else {
+    ti = tile % nt;
+    tj = tile / nt;
+  }
+  const int64_t p0 = chunk * kc, p1 = min(N, p0 + kc);
+  const int64_t q = ((p1 - p0 + 63) / 64) * 16;  // points per wave, whole steps
+  const int64_t w0 = p0 + wv * q, w1 = min(p1, w0 + q);
+  const double *pa[TI], *pb[TI];
+#pragma unroll
+  for (int r = 0; r < TI; ++r) {  // bands past the last repeat it; their sums are not written
+    pa[r] = A + int64_t(min(ti * T + 16 * r + lo, nb - 1)) * N + 4 * hi;
+    pb[r] = B + int64_t(min(tj * T + 16 * r + lo, nb - 1)) * N + 4 * hi;
+  }
+  V4 acc[TI][TI];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TI; ++j) acc[i][j] = V4{0.0, 0.0, 0.0, 0.0};
+  V4 a[2][TI], b[2][TI];
+  auto load = [&](V4 (&da)[TI], V4 (&db)[TI], int64_t p) {
+#pragma unroll
+    for (int r = 0; r < TI; ++r) {
+      da[r] = *reinterpret_cast<const U4 *>(pa[r] + p);
+      db[r] = *reinterpret_cast<const U4 *>(pb[r] + p);
+    }
+  };
+  auto mult = [&](const V4 (&da)[TI], const V4 (&db)[TI]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(db[j][k], da[i][k], acc[i][j], 0, 0, 0);
+  };
+  int64_t p = w0;
+  const int64_t full = w1 > w0 ? w0 + (w1 - w0) / 16 * 16 : w0;  // whole steps inside the band
+  if (p < full) load(a[0], b[0], p);
+  while (p < full) {
+    if (p + 16 < full) load(a[1], b[1], p + 16);
+    mult(a[0], b[0]);
+    p += 16;
+    if (p >= full) break;
+    if (p + 16 < full) load(a[0], b[0], p + 16);
+    mult(a[1], b[1]);
+    p += 16;
+  }
+  if (p < w1) {  // fewer than 16 points: point by point, zeros past the end
+#pragma unroll
+    for (int r = 0; r < TI; ++r)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const bool in = p + 4 * hi + k < w1;
+        const int64_t o = in ? p + k : p - 4 * hi;  // p itself is inside
+        a[0][r][k] = in ? pa[r][o] : 0.0;
+        b[0][r][k] = in ? pb[r][o] : 0.0;
+      }
+    mult(a[0], b[0]);
+  }
+  // lane (lo, hi) holds row lo of the columns 4 r + hi
+  __shared__ double red[T * T];  // the four waves' tiles, in wave order
+  for (int w = 1; w < 4; ++w) {
+    if (wv == w)
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TI; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) red[(16 * j + 4 * r + hi) * T + 16 * i + lo] = acc[i][j][r];
+    __syncthreads();
+    if (wv == 0)
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TI; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[i][j][r] += red[(16 * j + 4 * r + hi) * T + 16 * i + lo];
+    __syncthreads();
+  }
+  if (wv) return;
+  double *out = part + chunk * nb * nb;
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TI; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = ti * T + 16 * i + lo, col = tj * T + 16 * j + 4 * r + hi;
+        if (row < nb && col < nb) out[row + int64_t(col) * nb] = acc[i][j][r];
+      }
 }
 
-// C (nb x nb) = alpha A^T B with A, B column-major N x nb (leading dim N).
-// rocBLAS runs this K = N >> nb shape on a handful of output tiles (one
-// workgroup walks all of K when nb is small), so for nb <= 192 K is split
-// into chunks: one strided-batched GEMM into per-chunk partial matrices,
-// then a deterministic sum over the chunks.
-// Points per K chunk for an (N, nb) product: the autotuned choice if there
-// is one, else at most 256 chunks of >= 1024 points for nb <= 192 and one
-// GEMM above; 0 = one GEMM.
-int64_t gram_chunk(const rsg_ctx *ctx, int nb, int64_t N) {
+// C = alpha * the sum of nch partial matrices, eight threads per element;
+// sym: elements i <= j are given and written to both triangles
+__global__ __launch_bounds__(256) void k_gram_sum(const double *__restrict__ part, int64_t nch, int nb, int sym,
+                                                  double alpha, double *__restrict__ C) {
+  __shared__ double red[8][32];
+  const int64_t mat = int64_t(nb) * nb, t = int64_t(blockIdx.x) * 32 + threadIdx.x % 32;
+  const int c0 = threadIdx.x / 32;
+  const int i = int(t % nb), j = int(t / nb);
+  const bool act = t < mat && (!sym || i <= j);
+  double v = 0.0;
+  if (act)
+#pragma unroll 4
+    for (int64_t c = c0; c < nch; c += 8) v += part[c * mat + t];
+  red[c0][threadIdx.x % 32] = v;
+  __syncthreads();
+  if (c0 || !act) return;
+#pragma unroll
+  for (int k = 1; k < 8; ++k) v += red[k][threadIdx.x % 32];
+  C[t] = alpha * v;
+  if (sym) C[j + int64_t(i) * nb] = alpha * v;
+}
+
+// Bands per tile side: 32 or 48, whichever pads less (48 reads less per
+// product and takes ties).
+inline int gram_tile(int nb) { return (nb + 47) / 48 * 48 <= (nb + 31) / 32 * 32 ? 48 : 32; }
+
+// Where k_gram runs (us per product, against rocBLAS batched over chunks of
+// points and the sum of their results): 36^3, 20 bands 13 (35), 48^3, 40
+// bands 25 (52), 58^3, 77 bands 75 (184), U^T U of 72^3, 160 bands 335
+// (492).  rocBLAS's tiles are 128 bands a side, so it is the faster from 97
+// to 128 bands (72^3, 128: 209 against 253) and for the product of two
+// different blocks above (160 bands: 492 against 584).
+inline bool gram_own(int nb, bool sym) { return nb <= 96 || (sym && nb > 128 && nb <= 192); }
+
+// Points per chunk of an (N, nb) product: the autotuned choice if there is
+// one (0 = one GEMM), else
+// - k_gram: a block per CU, of 512 points or more (36^3, 20 bands: 13 us
+//   with 91 blocks, 22 with 32, 67 with 8);
+// - rocBLAS, which runs this K = N >> nb shape on a handful of output tiles:
+//   at most 256 chunks of 1024 points or more up to 192 bands, one GEMM
+//   above.
+int64_t gram_chunk(const rsg_ctx *ctx, int nb, int64_t N, bool sym) {
   for (const auto &e : ctx->gram_split)
     if (e[0] == N && e[1] == nb) return e[2];
-  if (nb > 192 || N < 4096) return 0;
-  return std::max<int64_t>(1024, (N + 255) / 256);
+  if (!gram_own(nb, sym)) return nb > 192 || N < 4096 ? 0 : std::max<int64_t>(1024, (N + 255) / 256);
+  const int64_t nt = (nb + gram_tile(nb) - 1) / gram_tile(nb), tiles = sym ? nt * (nt + 1) / 2 : nt * nt;
+  const int64_t nch = std::max<int64_t>(1, 256 / tiles);
+  return std::max<int64_t>(512, (N + nch - 1) / nch);
 }
 
 int gemm_tn_gram(rsg_ctx *ctx, int nb, int64_t N, double alpha, const double *A, const double *B, double *C,
                  int64_t kc_force = -1) {
   const double zero = 0.0, one = 1.0;
-  const int64_t kc = kc_force >= 0 ? kc_force : gram_chunk(ctx, nb, N);
-  if (kc <= 0 || kc >= N) {
+  const bool sym = A == B, own = gram_own(nb, sym);
+  const int64_t kc = kc_force >= 0 ? kc_force : gram_chunk(ctx, nb, N, sym);
+  if (kc <= 0 || (kc >= N && !own)) {
     RSG_BLAS_GUARDED(rocblas_dgemm(ctx->blas, rocblas_operation_transpose, rocblas_operation_none, nb, nb, int(N), &alpha, A,
                            int(N), B, int(N), &zero, C, nb));
     return RSG_OK;
   }
-  const int nfull = int(N / kc);
-  const int64_t krem = N - int64_t(nfull) * kc;
-  const int nbat = nfull + (krem > 0 ? 1 : 0);
-  const size_t mat = size_t(nb) * nb;
-  if (ctx->grampart.ensure(mat * nbat * sizeof(double)) != hipSuccess)
+  const int64_t mat = int64_t(nb) * nb, nch = (N + kc - 1) / kc;
+  if (ctx->grampart.ensure(size_t(mat) * nch * sizeof(double)) != hipSuccess)
     return ctx->fail(RSG_ERR_HIP, "gram product: scratch allocation failed");
   double *part = ctx->grampart.as<double>();
-  RSG_BLAS_GUARDED(rocblas_dgemm_strided_batched(ctx->blas, rocblas_operation_transpose, rocblas_operation_none, nb, nb,
-                                         int(kc), &one, A, int(N), kc, B, int(N), kc, &zero, part, nb,
-                                         rocblas_stride(mat), nfull));
-  if (krem > 0)
-    RSG_BLAS_GUARDED(rocblas_dgemm(ctx->blas, rocblas_operation_transpose, rocblas_operation_none, nb, nb, int(krem), &one,
-                           A + int64_t(nfull) * kc, int(N), B + int64_t(nfull) * kc, int(N), &zero,
-                           part + mat * nfull, nb));
-  const int count = int(mat);
-  hipLaunchKernelGGL(k_sum_batches, dim3((count + 255) / 256), dim3(256), 0, ctx->stream, part, nbat, count, alpha, C);
+  if (own) {
+    const int T = gram_tile(nb), nt = (nb + T - 1) / T, ntile = sym ? nt * (nt + 1) / 2 : nt * nt;
+    if (ntile * nch > 0x7fffffff) return ctx->fail(RSG_ERR_UNSUPPORTED, "gram product: too many workgroups");
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(unsigned(ntile * nch)), dim3(256), 0, ctx->stream, A, B, N, nb, kc, nt, ntile,
+                         part);
+    };
+    if (T == 48)
+      sym ? go(k_gram<3, true>) : go(k_gram<3, false>);
+    else
+      sym ? go(k_gram<2, true>) : go(k_gram<2, false>);
+  } else {
+    const int64_t nfull = N / kc, krem = N - nfull * kc;
+    RSG_BLAS_GUARDED(rocblas_dgemm_strided_batched(ctx->blas, rocblas_operation_transpose, rocblas_operation_none, nb, nb,
+                                           int(kc), &one, A, int(N), kc, B, int(N), kc, &zero, part, nb,
+                                           rocblas_stride(mat), int(nfull)));
+    if (krem > 0)
+      RSG_BLAS_GUARDED(rocblas_dgemm(ctx->blas, rocblas_operation_transpose, rocblas_operation_none, nb, nb, int(krem), &one,
+                             A + nfull * kc, int(N), B + nfull * kc, int(N), &zero, part + mat * nfull, nb));
+  }
+  hipLaunchKernelGGL(k_gram_sum, dim3(unsigned((mat + 31) / 32)), dim3(256), 0, ctx->stream, part, nch, nb,
+                     own && sym ? 1 : 0, alpha, C);
   RSG_HIP(hipGetLastError());
   return RSG_OK;
 }
@@ -1679,7 +1833,9 @@ __global__ void k_sum_batches_f32(const float *__restrict__ part, int nbat, int 
 // the chunk sum in FP64.
 int gemm_tn_gram_f32(rsg_ctx *ctx, int nb, int64_t N, double alpha, const float *A, const float *B, double *C) {
   const float zero = 0.f, one = 1.f;
-  int64_t kc = gram_chunk(ctx, nb, N);
+  int64_t kc = nb > 192 || N < 4096 ? 0 : std::max<int64_t>(1024, (N + 255) / 256);
+  for (const auto &e : ctx->gram_split)
+    if (e[0] == N && e[1] == nb) kc = e[2];
   if (kc <= 0 || kc > 16384) kc = std::min<int64_t>(N, 16384);
   const int nfull = int(N / kc);
   const int64_t krem = N - int64_t(nfull) * kc;
@@ -1723,6 +1879,10 @@ int autotune_gram(rsg_ctx *ctx, int nb, int reps, float *best_ms, int64_t *best_
   std::vector<int64_t> cand{0};
   for (int c = 8; c <= 512; c *= 2)
     if (N / c >= 512) cand.push_back((N + c - 1) / c);
+  if (gram_own(nb, true)) {
+    const int64_t kc = gram_chunk(ctx, nb, N, true);
+    if (kc > 0 && kc < N) cand.push_back(kc);
+  }
   hipEvent_t e0 = nullptr, e1 = nullptr;
   int rc = RSG_OK;
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) rc = RSG_ERR_HIP;

@@ -597,3 +597,32 @@ def test_conjugate_gradient_step_counts_and_grid_sizes(orc, ngrid, ncg):
     np.testing.assert_allclose(esp, esp_want, atol=1e-9)
     np.testing.assert_allclose(res, res_want, rtol=1e-7, atol=1e-12)
     assert np.abs(ctx.download_bands() - u_want).max() < 1e-7 * np.abs(u_want).max()
+
+
+@pytest.mark.parametrize("nb", [1, 16, 33, 48, 49, 96, 97, 131])
+@pytest.mark.parametrize("ngrid", [(13, 11, 9), (16, 16, 16)])
+def test_gram_products_over_band_counts(orc, ngrid, nb):
+    """The matrix-core Gram products at the edges of their band tiles, at the
+    rocBLAS range between, and over point counts that leave a remainder (odd
+    band starts) or none: orthonormal bands against the oracle's, and the
+    subspace eigenvalues (the product of two different blocks) against
+    LAPACK on the oracle's H psi.  Sums of up to 4096 terms in another order:
+    1e-12 of the largest value, eigenvalues 1e-12 of the largest |H|."""
+    from rsdft_develop_amd import gpu
+
+    base = systems.silicon_supercell(1, displacement=0.05, seed=4)
+    cell = systems.Cell(aa=np.diag([0.3 * n for n in ngrid]), frac=base.frac, kind=base.kind, species=base.species,
+                        ngrid=ngrid, nband=nb, md=6)
+    v = systems.model_vloc(cell)
+    ham = orc.Ham(cell, vloc=v)
+    ctx = gpu.Context().setup(cell, v)
+    u0 = systems.random_bands(cell.npoints, nb, seed=nb)
+    _load(ctx, u0)
+    print(f"case: Gram products {ngrid}, {nb} bands", flush=True)
+    ctx.gram_schmidt()
+    q = ctx.download_bands()
+    assert np.abs(q.T @ q * ham.dv - np.eye(nb)).max() < 1e-12
+    assert np.abs(q - ham.gram_schmidt(u0, "lusl")).max() < 1e-10
+    h = q.T @ ham.hpsi(q) * ham.dv
+    want = np.linalg.eigvalsh(0.5 * (h + h.T))
+    assert np.abs(ctx.subspace_diag() - want).max() < 1e-12 * np.abs(want).max()
