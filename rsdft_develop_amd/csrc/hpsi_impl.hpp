@@ -905,6 +905,7 @@ template <> HpsiShape &shape_of<float>(rsg_ctx *ctx) { return ctx->shape32; }
 
 constexpr size_t kMaxDynLds = 64 * 1024;
 constexpr int kCus = 256;      // compute units
+constexpr int64_t kSmallCall = int64_t(1) << 20;  // points times bands below which a stencil thread takes one row
 constexpr int kRunStart = 10;  // planes' worth of time a z-run's ring fill takes
 
 inline int round64(int v) { return (v + 63) / 64 * 64; }
@@ -950,7 +951,10 @@ int pick_ty_parts(int n1, int n2, int md, size_t s) {
 }
 
 // Tile rows per workgroup for ry rows per thread: balance idle lanes, the
-// partial last tile and the halo rows each plane re-reads.
+// partial last tile and the halo rows each plane re-reads.  FP64 with two
+// rows a thread spills beyond two halo elements per thread (75^3, 60 bands:
+// H psi 592 to 657 us there, 403 with 12 rows and 1.8): only if nothing
+// else fits.
 int pick_ty(int n1, int n2, int md, int ry, size_t s) {
   int best_ty = 0;
   double best = 1e300;
@@ -962,7 +966,8 @@ int pick_ty(int n1, int n2, int md, int ry, size_t s) {
     if (2 * md * n1 > 4 * round64(th)) continue;
     const int tiles = (n2 + ty - 1) / ty;
     const double cost = double(round64(th)) / th * double(tiles * ty) / n2 *
-                        (1.0 + 0.5 * 2.0 * md / ty) * (th < 128 ? 2.0 : 1.0);
+                        (1.0 + 0.5 * 2.0 * md / ty) * (th < 128 ? 2.0 : 1.0) *
+                        (s == sizeof(double) && ry == 2 && 2 * md * n1 > 2 * round64(th) ? 4.0 : 1.0);
     if (cost < best) {
       best = cost;
       best_ty = ty;
@@ -1124,7 +1129,12 @@ int launch_stencil(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, cons
 //   bands, two halo elements: 604 with two, 660 with one); there the rows go
 //   in parts where n1 is even (k_stencil's figures), and full rows stay for
 //   an odd n1, whose parts start misaligned (99^3, 240 bands: 3782 with full
-//   rows, 4001 with parts; 111 x 107 x 101: 4638 and 4762);
+//   rows, 4001 with parts; 111 x 107 x 101: 4638 and 4762).  More than 1.3
+//   padded rows cost more than the second row a thread gives (75 x 38 x 70,
+//   77 bands, 1.26: 252 with two, 258 with one);
+//   a call of few points is a chain of latencies, shorter with one row a
+//   thread (24^3, 12 bands: 27.0 with two, 24.7 with one; 36^3, 20 bands
+//   38.2 and 35.3; 40^3, 27 bands 45 either way);
 // - FP32 takes the pair kernel where it fits (72^3, 160 bands: 330 against
 //   395; 108^3, 480 bands: 3800 against 4400);
 // - the analytic form runs all bands at once (72^3, 160 bands FP64 in
@@ -1161,10 +1171,13 @@ HpsiShape resolve_shape(const rsg_ctx *ctx, const HpsiShape &in, size_t s, int n
   auto ty_bad = [&]() { return !row_tile(n1, ctx->md, sh.ry, sh.ty, s).fits; };
   if (sh.rx == 1 && auto_ry && s == sizeof(double)) {
     const int ty = ty_bad() ? pick_ty(n1, n2, ctx->md, 2, s) : sh.ty;
-    if (ty == 0 || (row_tile(n1, ctx->md, 2, ty, s).halo > 2 * row_tile(n1, ctx->md, 2, ty, s).threads)) {
+    const RowTile rt = row_tile(n1, ctx->md, 2, ty, s);
+    if (ty == 0 || rt.halo > 2 * rt.threads || (ty_bad() && (n2 + ty - 1) / ty * ty > 1.3 * n2)) {
       const int part = ty && n1 % 2 == 0 ? pick_ty_parts(n1, n2, ctx->md, s) : 0;
       if (part) sh.ty = part;
       else sh.ry = 1;
+    } else if (ctx->N * int64_t(nb) < kSmallCall) {
+      sh.ry = 1;
     }
   }
   if (sh.rx == 1 && ty_bad()) {
