@@ -9,6 +9,7 @@
 #include <string>
 #include <vector>
 
+#include "hpsi_shape.hpp"
 #include "rsdft_gpu.h"
 
 namespace rsg {
@@ -151,23 +152,6 @@ struct AnalyticGroups {
   int S = 0;  // n1 + n2 + n3
   std::vector<AnalyticGroup> g;  // atoms with projectors, in atom order
 };
-
-// Launch shape of the hpsi kernels for one grid and precision.  A zero ry,
-// ty, zlen, chunk, bt, rx or psplit is derived per call (resolve_shape).
-struct HpsiShape {
-  int ry = 0;     // rows per thread (y register blocking)
-  int ty = 0;     // rows per workgroup tile
-  int zlen = 0;   // z-planes per workgroup
-  int chunk = 0;  // bands per chunk (gather -> scatter -> stencil)
-  int bt = 0;     // bands per scatter thread / 4 * bt bands per apply wave
-  int order = 0;  // analytic projectors: 0 = nonlocal writes, stencil adds; 1 = stencil writes, nonlocal adds
-  int rx = 0;     // x-points per stencil thread: 1, or 2 (pair kernel: FP32, Md 6, even n1, ty | n2)
-  int proj = 0;   // analytic projections: 0 = per sphere segment (k_proj_m), 1 = by row tiles (k_proj_rows)
-  int plds = 0;   // KiB of LDS reserved per segment-projection wave (fewer waves in flight: a smaller L2 set)
-  int psplit = 0; // segment projections: pieces per segment (1, 2, 4, 8), each its own wave and partial slot
-};
-// pieces per segment where none are asked for
-constexpr int kAutoPieces = 4;
 
 // Learned preconditioner state: bf16 weight matrices for the kernels, the
 // FP32 master parameters with Adam moments, the normalised potential and

@@ -903,103 +903,18 @@ template <typename T> HpsiShape &shape_of(rsg_ctx *ctx);
 template <> HpsiShape &shape_of<double>(rsg_ctx *ctx) { return ctx->shape64; }
 template <> HpsiShape &shape_of<float>(rsg_ctx *ctx) { return ctx->shape32; }
 
-constexpr size_t kMaxDynLds = 64 * 1024;
-constexpr int kCus = 256;      // compute units
-constexpr int64_t kSmallCall = int64_t(1) << 20;  // points times bands below which a stencil thread takes one row
-constexpr int kRunStart = 10;  // planes' worth of time a z-run's ring fill takes
-
-inline int round64(int v) { return (v + 63) / 64 * 64; }
-
-// Workgroup of the one-point kernel for ty tile rows: full x-rows while 512
-// threads cover them, else (FP64, two rows a thread) the rows in nx equal
-// parts, whose columns beside the part are halo too.
-struct RowTile {
-  int nx, xw, threads, halo;  // halo elements per plane
-  size_t lds;
-  bool fits;
-};
-RowTile row_tile(int n1, int md, int ry, int ty, size_t s) {
-  RowTile r{1, n1, 0, 0, 0, false};
-  if (ry < 1 || ty < ry || ty % ry || ty / ry > 512 || n1 > 512) return r;
-  const int G = ty / ry;
-  while (r.xw * G > 512) ++r.nx, r.xw = (n1 + r.nx - 1) / r.nx;
-  const bool parts = r.nx > 1;
-  r.threads = round64(r.xw * G);
-  r.halo = 2 * md * (parts ? r.xw + ty : n1);
-  r.lds = (2 * size_t(ty + 2 * md) * (parts ? r.xw + 2 * md : n1) + 64) * s;
-  r.fits = r.lds <= kMaxDynLds &&
-           (parts ? s == sizeof(double) && ry == 2 && r.halo <= 2 * r.threads : r.halo <= 4 * r.threads);
-  return r;
-}
-
-// Tile rows for rows in parts: 16 to 20, with the least padding (8 to 14
-// rows leave more halo, 24 and more make the parts narrow: 144^3, 300 bands
-// 11.8 ms with 12 rows, 10.8 with 16, 11.9 with 24, 13.7 with 32).
-int pick_ty_parts(int n1, int n2, int md, size_t s) {
-  int best_ty = 0;
-  double best = 1e300;
-  for (int ty = 16; ty <= 20; ty += 2) {
-    const RowTile r = row_tile(n1, md, 2, ty, s);
-    if (!r.fits || r.nx == 1) continue;
-    const double cost = double(r.nx) * r.xw / n1 * double((n2 + ty - 1) / ty * ty) / n2;
-    if (cost < best) {
-      best = cost;
-      best_ty = ty;
-    }
-  }
-  return best_ty;
-}
-
-// Tile rows per workgroup for ry rows per thread: balance idle lanes, the
-// partial last tile and the halo rows each plane re-reads.  FP64 with two
-// rows a thread spills beyond two halo elements per thread (75^3, 60 bands:
-// H psi 592 to 657 us there, 403 with 12 rows and 1.8): only if nothing
-// else fits.
-int pick_ty(int n1, int n2, int md, int ry, size_t s) {
-  int best_ty = 0;
-  double best = 1e300;
-  for (int G = 1; n1 * G <= 512; ++G) {
-    const int ty = G * ry;
-    if (ty > ((n2 + ry - 1) / ry) * ry) break;
-    if ((2 * size_t(ty + 2 * md) * n1 + 64) * s > kMaxDynLds) break;
-    const int th = n1 * G;
-    if (2 * md * n1 > 4 * round64(th)) continue;
-    const int tiles = (n2 + ty - 1) / ty;
-    const double cost = double(round64(th)) / th * double(tiles * ty) / n2 *
-                        (1.0 + 0.5 * 2.0 * md / ty) * (th < 128 ? 2.0 : 1.0) *
-                        (s == sizeof(double) && ry == 2 && 2 * md * n1 > 2 * round64(th) ? 4.0 : 1.0);
-    if (cost < best) {
-      best = cost;
-      best_ty = ty;
-    }
-  }
-  return best_ty;
-}
-
-// Pair kernel (two x-points per thread): tile rows for ry rows per
-// thread among the divisors of n2, same cost model as pick_ty.
-constexpr int kPairMd = 6;
-
-inline bool pair_fits(int n1, int n2, int md, int ry, int ty, size_t s) {
-  if (md != kPairMd || n1 % 2 || n1 < 2 * md || ty <= 0 || ty % ry || n2 % ty) return false;
-  const int th = round64((n1 / 2) * (ty / ry));
-  const size_t lds = (2 * size_t(ty + 2 * md) * (n1 + 2 * md) + 128) * s;
-  return th <= 512 && lds <= kMaxDynLds && 2 * md * (n1 / 2) <= 4 * th;
-}
-
-int pick_ty_pair(int n1, int n2, int md, int ry, size_t s) {
-  int best_ty = 0;
-  double best = 1e300;
-  for (int ty = ry; ty <= n2; ty += ry) {
-    if (!pair_fits(n1, n2, md, ry, ty, s)) continue;
-    const int th = (n1 / 2) * (ty / ry);
-    const double cost = double(round64(th)) / th * (1.0 + 0.5 * 2.0 * md / ty) * (th < 128 ? 2.0 : 1.0);
-    if (cost < best) {
-      best = cost;
-      best_ty = ty;
-    }
-  }
-  return best_ty;
+// what resolve_shape needs; nonlocal: the call has a nonlocal part
+HpsiGrid shape_grid(const rsg_ctx *ctx, bool nonlocal) {
+  HpsiGrid g;
+  g.n1 = ctx->n[0];
+  g.n2 = ctx->n[1];
+  g.n3 = ctx->n[2];
+  g.md = ctx->md;
+  g.N = ctx->N;
+  g.nonlocal = nonlocal;
+  g.analytic = nonlocal && ctx->nl_mode != 1 && ctx->have_ana;
+  g.nseg = ctx->ana64.nseg;
+  return g;
 }
 
 template <int RY, int HM>
@@ -1120,131 +1035,6 @@ int launch_stencil(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, cons
   }
 }
 
-// Complete a launch shape: fields left at zero are derived from the grid,
-// the precision and the number of bands of the call.  Where the lines lie
-// (us per H psi call, analytic projectors):
-// - rows per thread: two share their y-window, but in FP64 with more than
-//   two halo elements per thread the registers no longer hold the prefetch
-//   (108^3, 480 bands: 11740 with two full rows, 7060 with one; 72^3, 160
-//   bands, two halo elements: 604 with two, 660 with one); there the rows go
-//   in parts where n1 is even (k_stencil's figures), and full rows stay for
-//   an odd n1, whose parts start misaligned (99^3, 240 bands: 3782 with full
-//   rows, 4001 with parts; 111 x 107 x 101: 4638 and 4762).  More than 1.3
-//   padded rows cost more than the second row a thread gives (75 x 38 x 70,
-//   77 bands, 1.26: 252 with two, 258 with one);
-//   a call of few points is a chain of latencies, shorter with one row a
-//   thread (24^3, 12 bands: 27.0 with two, 24.7 with one; 36^3, 20 bands
-//   38.2 and 35.3; 40^3, 27 bands 45 either way);
-// - FP32 takes the pair kernel where it fits (72^3, 160 bands: 330 against
-//   395; 108^3, 480 bands: 3800 against 4400);
-// - the analytic form runs all bands at once (72^3, 160 bands FP64 in
-//   chunks of 22: 1160, of 80: 709, whole: 618), its partial projections
-//   within 1 GiB;
-// - four pieces per segment (72^3 FP64, whole: 660 with one, 618 with four;
-//   36^3, 20 bands: 52 and 41);
-// - bands per apply wave: the least padding, then the most bands (160
-//   bands: 80 a wave 604, 32 a wave 620);
-// - z-runs: a run of zlen planes costs zlen + kRunStart planes' time (ring
-//   fill; 40^3, 27 bands: stencil 44, 27, 18 us in runs of 40, 20, 10), and
-//   the blocks go in rounds of as many as the CUs hold at once; the number
-//   of runs with the least rounds x run cost is taken (40^3, 27 bands: 216
-//   blocks 48.5, 270 blocks, so two rounds, 59.0; 24^3, 12 bands: one run
-//   34, six 26).
-HpsiShape resolve_shape(const rsg_ctx *ctx, const HpsiShape &in, size_t s, int nb, bool chunked) {
-  HpsiShape sh = in;
-  const int n1 = ctx->n[0], n2 = ctx->n[1], n3 = ctx->n[2];
-  if (sh.rx == 0) sh.rx = s == sizeof(float) ? 2 : 1;
-  bool auto_ry = sh.ry < 1 || sh.ry > 2;
-  if (auto_ry) sh.ry = 2;
-  if (sh.rx == 2) {  // pair kernel: FP32 only; else the one-point kernel
-    if (s != sizeof(float)) sh.rx = 1;
-    else if (!pair_fits(n1, n2, ctx->md, sh.ry, sh.ty, s)) {
-      int ty = pick_ty_pair(n1, n2, ctx->md, sh.ry, s);
-      if (ty == 0 && auto_ry) ty = pick_ty_pair(n1, n2, ctx->md, sh.ry = 1, s);
-      if (ty == 0) sh.rx = 1;
-      else sh.ty = ty;
-    }
-    if (sh.rx == 1 && auto_ry) sh.ry = 2;
-  } else {
-    sh.rx = 1;
-  }
-  auto ty_bad = [&]() { return !row_tile(n1, ctx->md, sh.ry, sh.ty, s).fits; };
-  if (sh.rx == 1 && auto_ry && s == sizeof(double)) {
-    const int ty = ty_bad() ? pick_ty(n1, n2, ctx->md, 2, s) : sh.ty;
-    const RowTile rt = row_tile(n1, ctx->md, 2, ty, s);
-    if (ty == 0 || rt.halo > 2 * rt.threads || (ty_bad() && (n2 + ty - 1) / ty * ty > 1.3 * n2)) {
-      const int part = ty && n1 % 2 == 0 ? pick_ty_parts(n1, n2, ctx->md, s) : 0;
-      if (part) sh.ty = part;
-      else sh.ry = 1;
-    } else if (ctx->N * int64_t(nb) < kSmallCall) {
-      sh.ry = 1;
-    }
-  }
-  if (sh.rx == 1 && ty_bad()) {
-    sh.ty = pick_ty(n1, n2, ctx->md, sh.ry, s);
-    if (sh.ty == 0) {
-      sh.ry = 1;
-      sh.ty = pick_ty(n1, n2, ctx->md, 1, s);
-    }
-  }
-  if (sh.psplit != 1 && sh.psplit != 2 && sh.psplit != 4 && sh.psplit != 8) sh.psplit = kAutoPieces;
-  const bool analytic = chunked && ctx->nl_mode != 1 && ctx->have_ana;
-  if (sh.chunk <= 0) {
-    sh.chunk = nb;
-    if (analytic) {
-      const size_t per_band = size_t(std::max(1, ctx->ana64.nseg)) * sh.psplit * 4 * s;
-      sh.chunk = int(std::min<size_t>(size_t(nb), std::max<size_t>(1, (size_t(1) << 30) / per_band)));
-      const int nch = (nb + sh.chunk - 1) / sh.chunk;
-      sh.chunk = (nb + nch - 1) / nch;  // chunks of equal size
-    } else if (chunked) {
-      // table form: psi + H psi of one chunk within ~128 MB of Infinity Cache
-      sh.chunk = int(std::max<size_t>(1, (size_t(64) << 20) / (size_t(ctx->N) * s)));
-    }
-  }
-  sh.chunk = std::max(1, std::min(sh.chunk, nb));
-  if (sh.zlen <= 0) {
-    int tiles = (n2 + sh.ty - 1) / sh.ty, waves, per_cu;
-    if (sh.rx == 2) {
-      waves = round64((n1 / 2) * (sh.ty / sh.ry)) / 64;
-      per_cu = sh.ry == 1 ? 12 : 8;
-    } else {
-      const RowTile rt = row_tile(n1, ctx->md, sh.ry, sh.ty, s);
-      tiles *= rt.nx;
-      waves = std::max(1, rt.threads / 64);
-      per_cu = sh.ry == 1 && rt.halo <= 2 * rt.threads ? 12 : 8;
-    }
-    const int64_t slots = int64_t(kCus) * std::max(1, per_cu / std::max(1, waves)), blocks = int64_t(tiles) * sh.chunk;
-    int64_t best = 0;
-    for (int zr = 1; zr <= std::max(1, n3 / 4); ++zr) {
-      const int zl = (n3 + zr - 1) / zr;
-      const int64_t cost = (blocks * ((n3 + zl - 1) / zl) + slots - 1) / slots * (zl + kRunStart);
-      if (!best || cost < best) {
-        best = cost;
-        sh.zlen = zl;
-      }
-      if (blocks * zr >= 8 * slots) break;
-    }
-  }
-  sh.zlen = std::max(1, std::min(sh.zlen, n3));
-  if (sh.bt != 4 && sh.bt != 8 && sh.bt != 16 && sh.bt != 20 && sh.bt != 32) {
-    sh.bt = 8;
-    if (analytic) {
-      int best = 0;
-      for (int bt : {20, 16, 8, 4}) {
-        const int pad = (sh.chunk + 4 * bt - 1) / (4 * bt) * (4 * bt);
-        if (!best || pad < best) {
-          best = pad;
-          sh.bt = bt;
-        }
-      }
-    }
-  }
-  if (sh.order != 0 && sh.order != 1) sh.order = 0;
-  if (sh.proj < 0 || sh.proj > 2) sh.proj = 0;
-  if (sh.plds < 0 || sh.plds > 64) sh.plds = 0;
-  return sh;
-}
-
 // dynamic LDS of k_proj_rows<T>: the staged rows of 16 bands (odd stride)
 // and the per-atom sums of the block
 template <typename T> size_t row_tiles_lds(const rsg_ctx *ctx, const AnalyticDev<T> &an) {
@@ -1294,7 +1084,7 @@ int launch_kinetic(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, int 
   if (nb == 0) return RSG_OK;
   if (nb > 65535) return ctx->fail(RSG_ERR_ARG, "op_kinetic: nb above 65535");
   if (!psi || !hpsi) return ctx->fail(RSG_ERR_ARG, "op_kinetic: null buffer");
-  const HpsiShape sh = resolve_shape(ctx, shape_of<T>(ctx), sizeof(T), nb, false);
+  const HpsiShape sh = resolve_shape(shape_grid(ctx, false), shape_of<T>(ctx), sizeof(T), nb);
   int rc = launch_stencil<T>(ctx, psi, hpsi, ld, nb, sh, accumulate ? 1 : 0);
   if (rc) return rc;
   hipError_t e = hipGetLastError();
@@ -1337,7 +1127,7 @@ int launch_hpsi(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, const H
   if (nb == 0) return RSG_OK;
   if (nb > 65535) return ctx->fail(RSG_ERR_ARG, "hpsi: nb above 65535");
   if (!psi || !hpsi) return ctx->fail(RSG_ERR_ARG, "hpsi: null buffer");
-  HpsiShape sh = resolve_shape(ctx, shape_of<T>(ctx), sizeof(T), nb, ctx->have_nl);
+  HpsiShape sh = resolve_shape(shape_grid(ctx, ctx->have_nl), shape_of<T>(ctx), sizeof(T), nb);
   if (!ctx->have_nl) {
     int rc = launch_stencil<T>(ctx, psi, hpsi, ld, nb, sh, 0);
     if (rc) return rc;
@@ -1456,7 +1246,7 @@ int resolved_shape(rsg_ctx *ctx, int precision, int nb, HpsiShape *out) {
   if (precision != 64 && precision != 32) return ctx->fail(RSG_ERR_ARG, "hpsi shape: precision must be 64 or 32");
   if (nb < 1) return ctx->fail(RSG_ERR_ARG, "hpsi shape: nb < 1");
   const size_t s = precision == 64 ? 8 : 4;
-  *out = resolve_shape(ctx, precision == 64 ? ctx->shape64 : ctx->shape32, s, nb, ctx->have_nl);
+  *out = resolve_shape(shape_grid(ctx, ctx->have_nl), precision == 64 ? ctx->shape64 : ctx->shape32, s, nb);
   return RSG_OK;
 }
 
@@ -1501,12 +1291,12 @@ template <typename T> int autotune_t(rsg_ctx *ctx, int nb, int reps, float *best
   // deterministic non-trivial content: timing does not depend on values
   (void)hipMemsetAsync(psi, 0x3f, bytes, ctx->stream);
   const size_t s = sizeof(T);
-  HpsiShape best = resolve_shape(ctx, HpsiShape(), s, nb, ctx->have_nl);
+  HpsiShape best = resolve_shape(shape_grid(ctx, ctx->have_nl), HpsiShape(), s, nb);
   float tbest = 0.f;
   int rc = time_shape<T>(ctx, psi, hpsi, nb, best, reps, &tbest);
   auto consider = [&](HpsiShape cand) {
     if (rc) return;
-    cand = resolve_shape(ctx, cand, s, nb, ctx->have_nl);
+    cand = resolve_shape(shape_grid(ctx, ctx->have_nl), cand, s, nb);
     float t = 0.f;
     int r = time_shape<T>(ctx, psi, hpsi, nb, cand, reps, &t);
     if (r == RSG_ERR_UNSUPPORTED) return;  // shape does not fit this grid

@@ -1,0 +1,48 @@
+"""Launch-shape rules of the H psi kernels (csrc/hpsi_shape.hpp), on the CPU.
+
+The rules are host code without a HIP call; tests/hpsi_shape_rules.cpp puts
+them behind a line protocol.  A shape is what the launch code takes: it has
+to fit the kernel it is for.
+"""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "rsdft_develop_amd", "csrc")
+FIELDS = ("ry", "ty", "zlen", "chunk", "bt", "rx", "psplit", "fits")
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("clang++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    exe = str(tmp_path_factory.mktemp("rules") / "hpsi_shape_rules")
+    subprocess.run([cxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-I", CSRC,
+                    os.path.join(HERE, "hpsi_shape_rules.cpp"), "-o", exe], check=True)
+
+    def ask(lines):
+        r = subprocess.run([exe], input="\n".join(lines) + "\n", capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, f"exit {r.returncode} after {len(r.stdout.splitlines())} of {len(lines)} answers"
+        return [dict(zip(FIELDS, map(int, a.split()))) for a in r.stdout.splitlines()]
+
+    return ask
+
+
+def _resolve(n, md=6, size=8, nb=64, nonlocal_=1, analytic=1, nseg=2000, **shape):
+    s = {k: shape.get(k, 0) for k in FIELDS[:-1]}
+    return (f"resolve {n[0]} {n[1]} {n[2]} {md} {size} {nb} {nonlocal_} {analytic} {nseg} "
+            f"{s['ry']} {s['ty']} {s['zlen']} {s['chunk']} {s['bt']} {s['rx']} {s['psplit']}")
+
+
+@pytest.mark.parametrize("size", [8, 4])
+def test_derived_shapes_fit_ordinary_grids(rules, size):
+    """Rows of 16 to 128 points with every finite-difference order whose halo
+    four elements a thread cover."""
+    grids = [(n1, n2, n3) for n1 in range(16, 129, 7) for n2 in (9, 24, 45, 108) for n3 in (3, 36, 99)]
+    ask = [(n, md, nb) for n in grids for md in (1, 4, 6, 8) for nb in (1, 37, 480)]
+    for (n, md, nb), sh in zip(ask, rules([_resolve(n, md=md, size=size, nb=nb) for n, md, nb in ask])):
+        assert sh["fits"] and 1 <= sh["zlen"] <= n[2] and 1 <= sh["chunk"] <= nb, (n, md, nb, sh)
