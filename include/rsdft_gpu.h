@@ -50,7 +50,11 @@ void *rsg_stream(rsg_ctx *ctx);
  * (rgrid_sol_module.f90:26-39: Hgrid, dV) and init_kinetic
  * (kinetic/kinetic_module.f90:28-180; get_coef_lapla_fd, fd_module.f90:18-54).
  * Orthorhombic cells only (the Gamma-path cross terms of
- * d_kinetic_sol_module.f90:351-529 vanish). */
+ * d_kinetic_sol_module.f90:351-529 vanish).
+ * Any n1 is taken here; H psi and the kinetic operator return
+ * RSG_ERR_UNSUPPORTED where no kernel takes the x-rows: in FP64 above 512
+ * points (128 with md 8), in FP32 above what one workgroup stages with its
+ * halo (170 points with md 6, up to 340 for even n1). */
 int rsg_set_grid(rsg_ctx *ctx, int n1, int n2, int n3, const double *aa,
                  int md);
 /* dv, hgrid[3], coef_lap0 and coef_lap[axis*md + m-1] as the context uses

@@ -917,6 +917,11 @@ HpsiGrid shape_grid(const rsg_ctx *ctx, bool nonlocal) {
   return g;
 }
 
+int no_stencil_tile(rsg_ctx *ctx) {
+  return ctx->fail(RSG_ERR_UNSUPPORTED, "hpsi: no stencil tile fits grid rows of " + std::to_string(ctx->n[0]) +
+                                            " points with md " + std::to_string(ctx->md));
+}
+
 template <int RY, int HM>
 int launch_stencil2_t(rsg_ctx *ctx, const float *psi, float *hpsi, int64_t ld, int nb, const HpsiShape &sh,
                       int accumulate) {
@@ -1085,6 +1090,7 @@ int launch_kinetic(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, int 
   if (nb > 65535) return ctx->fail(RSG_ERR_ARG, "op_kinetic: nb above 65535");
   if (!psi || !hpsi) return ctx->fail(RSG_ERR_ARG, "op_kinetic: null buffer");
   const HpsiShape sh = resolve_shape(shape_grid(ctx, false), shape_of<T>(ctx), sizeof(T), nb);
+  if (sh.ty == 0) return no_stencil_tile(ctx);
   int rc = launch_stencil<T>(ctx, psi, hpsi, ld, nb, sh, accumulate ? 1 : 0);
   if (rc) return rc;
   hipError_t e = hipGetLastError();
@@ -1128,6 +1134,7 @@ int launch_hpsi(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, const H
   if (nb > 65535) return ctx->fail(RSG_ERR_ARG, "hpsi: nb above 65535");
   if (!psi || !hpsi) return ctx->fail(RSG_ERR_ARG, "hpsi: null buffer");
   HpsiShape sh = resolve_shape(shape_grid(ctx, ctx->have_nl), shape_of<T>(ctx), sizeof(T), nb);
+  if (sh.ty == 0) return no_stencil_tile(ctx);
   if (!ctx->have_nl) {
     int rc = launch_stencil<T>(ctx, psi, hpsi, ld, nb, sh, 0);
     if (rc) return rc;
@@ -1247,7 +1254,7 @@ int resolved_shape(rsg_ctx *ctx, int precision, int nb, HpsiShape *out) {
   if (nb < 1) return ctx->fail(RSG_ERR_ARG, "hpsi shape: nb < 1");
   const size_t s = precision == 64 ? 8 : 4;
   *out = resolve_shape(shape_grid(ctx, ctx->have_nl), precision == 64 ? ctx->shape64 : ctx->shape32, s, nb);
-  return RSG_OK;
+  return out->ty == 0 ? no_stencil_tile(ctx) : RSG_OK;
 }
 
 namespace {

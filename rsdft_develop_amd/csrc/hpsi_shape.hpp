@@ -163,6 +163,10 @@ inline int pick_ty_pair(int n1, int n2, int md, int ry, size_t s) {
 //   of runs with the least rounds x run cost is taken (40^3, 27 bands: 216
 //   blocks 48.5, 270 blocks, so two rounds, 59.0; 24^3, 12 bands: one run
 //   34, six 26).
+// A shape with ty == 0 says that no kernel takes the grid's rows (the caller
+// refuses the call): full rows end at 170 points with md 6, where three tile
+// rows are the least that stage their halo and the most that 512 threads
+// cover, and only the FP64 kernel takes rows in parts.
 inline HpsiShape resolve_shape(const HpsiGrid &gr, const HpsiShape &in, size_t s, int nb) {
   HpsiShape sh = in;
   const int n1 = gr.n1, n2 = gr.n2, n3 = gr.n3;
@@ -199,7 +203,12 @@ inline HpsiShape resolve_shape(const HpsiGrid &gr, const HpsiShape &in, size_t s
       sh.ry = 1;
       sh.ty = pick_ty(n1, n2, gr.md, 1, s);
     }
+    if (sh.ty == 0 && s == sizeof(double)) {  // rows too long for whole ones, of any parity
+      sh.ry = 2;
+      sh.ty = pick_ty_parts(n1, n2, gr.md, s);
+    }
   }
+  if (sh.ty == 0) return sh;  // no tile fits
   if (sh.psplit != 1 && sh.psplit != 2 && sh.psplit != 4 && sh.psplit != 8) sh.psplit = kAutoPieces;
   if (sh.chunk <= 0) {
     sh.chunk = nb;

@@ -227,6 +227,36 @@ def test_stencil_rows_in_parts(orc, gpu_mod, ngrid, ty, zlen):
     np.testing.assert_array_equal(got, full)
 
 
+@pytest.mark.parametrize("ngrid,md", [((171, 24, 25), 6), ((172, 27, 24), 6), ((192, 25, 24), 7), ((256, 24, 24), 6)])
+def test_long_rows(orc, gpu_mod, ngrid, md):
+    """FP64 rows that only fit in parts (odd, even, md 7): H psi and the
+    local part alone against the oracle; FP32 rows with no kernel of their
+    own are refused by every entry point that needs a launch shape."""
+    from rsdft_develop_amd import hip
+
+    base = systems.silicon_supercell(1, displacement=0.1, seed=5)
+    cell = systems.Cell(aa=np.diag([0.3 * n for n in ngrid]), frac=base.frac, kind=base.kind, species=base.species,
+                        ngrid=ngrid, nband=2, md=md)
+    ham, ctx = _pair(orc, gpu_mod, cell)
+    psi = systems.random_bands(cell.npoints, 2, seed=ngrid[0])
+    print(f"case: long rows {ngrid} md {md}, shape {ctx.hpsi_shape(64, 2)}", flush=True)
+    _close(ctx.hamiltonian(psi), ham.hpsi(psi), 1e-12)
+    local = orc.Ham(cell, vloc=systems.model_vloc(cell), projectors=False)
+    d_in, d_out = hip.DeviceArray.from_numpy(psi), hip.DeviceArray(psi.shape)
+    ctx.op_kinetic_device(d_in.ptr, d_out.ptr, cell.npoints, 2)
+    ctx.synchronize()
+    _close(d_out.to_numpy(), local.hpsi(psi), 1e-12)
+    if ngrid[0] % 2 or md != 6:
+        f = lambda: ctx.hpsi_device(d_in.ptr, d_out.ptr, cell.npoints, 2, dtype=np.float32)  # noqa: E731
+        k = lambda: ctx.op_kinetic_device(d_in.ptr, d_out.ptr, cell.npoints, 2, dtype=np.float32)  # noqa: E731
+        for call in (f, k, lambda: ctx.hpsi_shape(32, 2), lambda: ctx.autotune_hpsi(32, 2, reps=1)):
+            with pytest.raises(gpu_mod.RSDFTGPUError) as e:
+                call()
+            assert e.value.code == 6
+    d_in.free()
+    d_out.free()
+
+
 def test_hpsi_errors(gpu_mod):
     ctx = gpu_mod.Context()
     a = np.zeros((8, 1), order="F")

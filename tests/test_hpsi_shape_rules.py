@@ -46,3 +46,19 @@ def test_derived_shapes_fit_ordinary_grids(rules, size):
     ask = [(n, md, nb) for n in grids for md in (1, 4, 6, 8) for nb in (1, 37, 480)]
     for (n, md, nb), sh in zip(ask, rules([_resolve(n, md=md, size=size, nb=nb) for n, md, nb in ask])):
         assert sh["fits"] and 1 <= sh["zlen"] <= n[2] and 1 <= sh["chunk"] <= nb, (n, md, nb, sh)
+
+
+def test_rows_too_long_for_whole_ones_go_in_parts(rules):
+    """FP64 rows above 170 points (md 6): three whole rows no longer stage
+    their halo in 512 threads, so every such row is split, odd ones too."""
+    ask = [((n1, n2, 20), md, ry) for n1 in (171, 172, 180, 192, 255, 256, 320, 511, 512) for n2 in (5, 24, 36)
+           for md in (6, 7) for ry in (0, 1, 2)]
+    for (n, md, ry), sh in zip(ask, rules([_resolve(n, md=md, ry=ry) for n, md, ry in ask])):
+        assert sh["fits"] and sh["ry"] == 2 and n[0] * sh["ty"] // 2 > 512, (n, md, ry, sh)
+
+
+@pytest.mark.parametrize("n,md,size", [((171, 24, 24), 6, 4), ((192, 25, 24), 5, 4), ((129, 24, 24), 8, 8),
+                                       ((513, 8, 8), 6, 8)])
+def test_rows_that_no_kernel_takes_have_no_tile(rules, n, md, size):
+    sh, = rules([_resolve(n, md=md, size=size)])
+    assert sh["ty"] == 0 and not sh["fits"]
