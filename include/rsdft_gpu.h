@@ -142,8 +142,9 @@ int rsg_hpsi_f64_host(rsg_ctx *ctx, const double *psi, double *hpsi,
  * nonlocal apply (4/8/16/20/32: 16, 32, 64, 80 or 128 bands per matrix-core
  * wave of the analytic form; the table form's scatter takes 4/8/16, and 8
  * for the others).  Zero fields (the default) are derived from the grid and
- * the bands of each call.  No reference
- * counterpart (launch tuning of this implementation). */
+ * the bands of each call; a ty that some kernel takes is used as given, with
+ * rows and points per thread that suit it where those are not set.  No
+ * reference counterpart (launch tuning of this implementation). */
 int rsg_set_hpsi_shape(rsg_ctx *ctx, int precision, int ry, int ty, int zlen,
                        int chunk, int bt);
 /* Order of the two passes over H psi with analytic projectors: 0 = the

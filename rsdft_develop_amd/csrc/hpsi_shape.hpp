@@ -170,33 +170,43 @@ inline int pick_ty_pair(int n1, int n2, int md, int ry, size_t s) {
 inline HpsiShape resolve_shape(const HpsiGrid &gr, const HpsiShape &in, size_t s, int nb) {
   HpsiShape sh = in;
   const int n1 = gr.n1, n2 = gr.n2, n3 = gr.n3;
-  if (sh.rx == 0) sh.rx = s == sizeof(float) ? 2 : 1;
-  bool auto_ry = sh.ry < 1 || sh.ry > 2;
-  if (auto_ry) sh.ry = 2;
-  if (sh.rx == 2) {  // pair kernel: FP32 only; else the one-point kernel
-    if (s != sizeof(float)) sh.rx = 1;
-    else if (!pair_fits(n1, n2, gr.md, sh.ry, sh.ty, s)) {
+  const bool auto_ry = sh.ry < 1 || sh.ry > 2;
+  const auto one_fits = [&](int ry) { return row_tile(n1, gr.md, ry, sh.ty, s).fits; };
+  const auto two_fits = [&](int ry) { return pair_fits(n1, n2, gr.md, ry, sh.ty, s); };
+  // tile rows that the caller gives stay where a kernel takes them, with the
+  // rows and points a thread that fit them
+  const bool one = auto_ry ? one_fits(2) || one_fits(1) : one_fits(sh.ry);
+  const bool two = auto_ry ? two_fits(2) || two_fits(1) : two_fits(sh.ry);
+  if (sh.rx == 0) sh.rx = s == sizeof(float) && (two || !one) ? 2 : 1;
+  if (sh.rx == 2 && s == sizeof(float)) {  // pair kernel: FP32 only; else the one-point kernel
+    if (auto_ry) sh.ry = two && !two_fits(2) ? 1 : 2;
+    if (!two) {
       int ty = pick_ty_pair(n1, n2, gr.md, sh.ry, s);
       if (ty == 0 && auto_ry) ty = pick_ty_pair(n1, n2, gr.md, sh.ry = 1, s);
       if (ty == 0) sh.rx = 1;
       else sh.ty = ty;
     }
-    if (sh.rx == 1 && auto_ry) sh.ry = 2;
   } else {
     sh.rx = 1;
   }
-  auto ty_bad = [&]() { return !row_tile(n1, gr.md, sh.ry, sh.ty, s).fits; };
-  if (sh.rx == 1 && auto_ry && s == sizeof(double)) {
-    const int ty = ty_bad() ? pick_ty(n1, n2, gr.md, 2, s) : sh.ty;
-    const RowTile rt = row_tile(n1, gr.md, 2, ty, s);
-    if (ty == 0 || rt.halo > 2 * rt.threads || (ty_bad() && (n2 + ty - 1) / ty * ty > 1.3 * n2)) {
-      const int part = ty && n1 % 2 == 0 ? pick_ty_parts(n1, n2, gr.md, s) : 0;
-      if (part) sh.ty = part;
-      else sh.ry = 1;
-    } else if (gr.N * int64_t(nb) < kSmallCall) {
-      sh.ry = 1;
+  if (sh.rx == 1 && auto_ry) {
+    sh.ry = one && !one_fits(2) ? 1 : 2;
+    if (s == sizeof(double) && sh.ry == 2) {
+      const int ty = one ? sh.ty : pick_ty(n1, n2, gr.md, 2, s);
+      const RowTile rt = row_tile(n1, gr.md, 2, ty, s);
+      const bool slow = ty == 0 || (rt.nx == 1 && rt.halo > 2 * rt.threads);  // full rows whose halo spills
+      if (one) {
+        if ((slow || gr.N * int64_t(nb) < kSmallCall) && one_fits(1)) sh.ry = 1;
+      } else if (slow || (n2 + ty - 1) / ty * ty > 1.3 * n2) {
+        const int part = ty && n1 % 2 == 0 ? pick_ty_parts(n1, n2, gr.md, s) : 0;
+        if (part) sh.ty = part;
+        else sh.ry = 1;
+      } else if (gr.N * int64_t(nb) < kSmallCall) {
+        sh.ry = 1;
+      }
     }
   }
+  const auto ty_bad = [&]() { return !one_fits(sh.ry); };
   if (sh.rx == 1 && ty_bad()) {
     sh.ty = pick_ty(n1, n2, gr.md, sh.ry, s);
     if (sh.ty == 0) {

@@ -62,3 +62,26 @@ def test_rows_too_long_for_whole_ones_go_in_parts(rules):
 def test_rows_that_no_kernel_takes_have_no_tile(rules, n, md, size):
     sh, = rules([_resolve(n, md=md, size=size)])
     assert sh["ty"] == 0 and not sh["fits"]
+
+
+@pytest.mark.parametrize("n,size,ty,rx", [
+    ((72, 72, 72), 4, 10, 1), ((72, 72, 72), 4, 14, 1),  # no divisor of n2: not for the pair kernel
+    ((72, 72, 72), 4, 12, 2), ((72, 72, 72), 4, 9, 2),   # divisors: the pair kernel, 9 with one row a thread
+    ((75, 38, 70), 4, 12, 1),                            # odd rows
+    ((108, 108, 108), 8, 4, 1), ((108, 108, 108), 8, 8, 1), ((144, 144, 144), 8, 3, 1),  # beside rows in parts
+    ((36, 36, 36), 8, 18, 1), ((36, 36, 36), 8, 9, 1),
+])
+def test_tile_rows_that_a_caller_sets_are_used(rules, n, size, ty, rx):
+    """With ry and rx left to the rules; a second answer with all three set
+    is the same."""
+    for nb in (2, 160):
+        sh, = rules([_resolve(n, size=size, ty=ty, nb=nb)])
+        assert (sh["ty"], sh["rx"], sh["fits"]) == (ty, rx, 1), sh
+        again, = rules([_resolve(n, size=size, ty=ty, nb=nb, ry=sh["ry"], rx=sh["rx"])])
+        assert again == sh
+
+
+def test_tile_rows_that_fit_no_kernel_are_replaced(rules):
+    for size in (8, 4):
+        sh, derived = rules([_resolve((72, 72, 72), size=size, ty=97), _resolve((72, 72, 72), size=size)])
+        assert sh == derived and sh["fits"]
