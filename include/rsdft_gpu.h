@@ -207,9 +207,11 @@ int rsg_autotune_hpsi(rsg_ctx *ctx, int precision, int nb, int reps,
 /* The Gram products U^T X (N x nb by N x nb, K = N) of Gram-Schmidt and
  * subspace_diag: time one rocBLAS GEMM over all of K against K-splits into
  * 8..512 chunks (the library's own kernel or a strided-batched GEMM, plus a
- * chunk sum), reps calls each on scratch bands, and keep the fastest for (N, nb) in this context.
- * chunk receives the points per chunk (0 = one GEMM); best_ms and chunk
- * may be NULL.  No reference counterpart (launch tuning). */
+ * chunk sum), reps calls each on scratch bands, and keep the fastest for
+ * (N, nb) in this context, separately for U^T U and for the product of two
+ * blocks where they run different kernels.  chunk receives the points per
+ * chunk of U^T U (0 = one GEMM); best_ms and chunk may be NULL.  No
+ * reference counterpart (launch tuning). */
 int rsg_autotune_gram(rsg_ctx *ctx, int nb, int reps, float *best_ms,
                       int64_t *chunk);
 

@@ -5,10 +5,10 @@
 #include <rocblas/rocblas.h>
 
 #include <cstdint>
-#include <array>
 #include <string>
 #include <vector>
 
+#include "gram_rules.hpp"
 #include "hpsi_shape.hpp"
 #include "rsdft_gpu.h"
 
@@ -270,9 +270,8 @@ struct rsg_ctx {
   int64_t cg_graph_launches = 0;   // band blocks run from a captured graph
   int64_t cg_graph_failures = 0;   // captures the runtime refused
   std::vector<rsg::CgGraph> cg_graph_cache;
-  // K-split of the U^T X Gram products chosen by the autotuner, per
-  // (N, nb): points per chunk, 0 = one GEMM over all of K
-  std::vector<std::array<int64_t, 3>> gram_split;
+  // K-splits of the Gram products chosen by the autotuner
+  std::vector<rsg::GramSplit> gram_split;
   rsg::DevBuf dead;                // store target of padding lanes (64 doubles)
   rsg::ScfState *scf = nullptr;    // density/potential state of the SCF step
   rsg::LpcState lpc;               // learned CG preconditioner

@@ -1751,39 +1751,13 @@ __global__ __launch_bounds__(256) void k_gram_sum(const double *__restrict__ par
   if (sym) C[j + int64_t(i) * nb] = alpha * v;
 }
 
-// Bands per tile side: 32 or 48, whichever pads less (48 reads less per
-// product and takes ties).
-inline int gram_tile(int nb) { return (nb + 47) / 48 * 48 <= (nb + 31) / 32 * 32 ? 48 : 32; }
-
-// Where k_gram runs (us per product, against rocBLAS batched over chunks of
-// points and the sum of their results): 36^3, 20 bands 13 (35), 48^3, 40
-// bands 25 (52), 58^3, 77 bands 75 (184), U^T U of 72^3, 160 bands 335
-// (492).  rocBLAS's tiles are 128 bands a side, so it is the faster from 97
-// to 128 bands (72^3, 128: 209 against 253) and for the product of two
-// different blocks above (160 bands: 492 against 584).
-inline bool gram_own(int nb, bool sym) { return nb <= 96 || (sym && nb > 128 && nb <= 192); }
-
-// Points per chunk of an (N, nb) product: the autotuned choice if there is
-// one (0 = one GEMM), else
-// - k_gram: a block per CU, of 512 points or more (36^3, 20 bands: 13 us
-//   with 91 blocks, 22 with 32, 67 with 8);
-// - rocBLAS, which runs this K = N >> nb shape on a handful of output tiles:
-//   at most 256 chunks of 1024 points or more up to 192 bands, one GEMM
-//   above.
-int64_t gram_chunk(const rsg_ctx *ctx, int nb, int64_t N, bool sym) {
-  for (const auto &e : ctx->gram_split)
-    if (e[0] == N && e[1] == nb) return e[2];
-  if (!gram_own(nb, sym)) return nb > 192 || N < 4096 ? 0 : std::max<int64_t>(1024, (N + 255) / 256);
-  const int64_t nt = (nb + gram_tile(nb) - 1) / gram_tile(nb), tiles = sym ? nt * (nt + 1) / 2 : nt * nt;
-  const int64_t nch = std::max<int64_t>(1, 256 / tiles);
-  return std::max<int64_t>(512, (N + nch - 1) / nch);
-}
-
 int gemm_tn_gram(rsg_ctx *ctx, int nb, int64_t N, double alpha, const double *A, const double *B, double *C,
                  int64_t kc_force = -1) {
   const double zero = 0.0, one = 1.0;
-  const bool sym = A == B, own = gram_own(nb, sym);
-  const int64_t kc = kc_force >= 0 ? kc_force : gram_chunk(ctx, nb, N, sym);
+  const bool sym = A == B;
+  const int form = sym ? kGramSame : kGramPair;
+  const bool own = gram_own(nb, form);
+  const int64_t kc = kc_force >= 0 ? kc_force : gram_chunk(ctx->gram_split, nb, N, form);
   if (kc <= 0 || (kc >= N && !own)) {
     RSG_BLAS_GUARDED(rocblas_dgemm(ctx->blas, rocblas_operation_transpose, rocblas_operation_none, nb, nb, int(N), &alpha, A,
                            int(N), B, int(N), &zero, C, nb));
@@ -1833,9 +1807,7 @@ __global__ void k_sum_batches_f32(const float *__restrict__ part, int nbat, int 
 // the chunk sum in FP64.
 int gemm_tn_gram_f32(rsg_ctx *ctx, int nb, int64_t N, double alpha, const float *A, const float *B, double *C) {
   const float zero = 0.f, one = 1.f;
-  int64_t kc = nb > 192 || N < 4096 ? 0 : std::max<int64_t>(1024, (N + 255) / 256);
-  for (const auto &e : ctx->gram_split)
-    if (e[0] == N && e[1] == nb) kc = e[2];
+  int64_t kc = gram_chunk(ctx->gram_split, nb, N, kGramF32);
   if (kc <= 0 || kc > 16384) kc = std::min<int64_t>(N, 16384);
   const int nfull = int(N / kc);
   const int64_t krem = N - int64_t(nfull) * kc;
@@ -1860,62 +1832,71 @@ int gemm_tn_gram_f32(rsg_ctx *ctx, int nb, int64_t N, double alpha, const float 
 }
 }  // namespace
 
-// Time one GEMM over all of K against K-splits into 8..512 chunks of at
-// least 512 points, for nb bands of the current grid (scratch bands, reps
-// calls each), and keep the fastest for (N, nb).  The products are the same
-// up to summation order.
+// Time one GEMM over all of K against K-splits (gram_candidates) for nb bands
+// of the current grid (scratch bands, reps calls each), and keep the fastest
+// for (N, nb): the product of one block with itself, and that of two blocks
+// where another kernel runs it.  The products are the same up to summation
+// order.  best_ms and best_kc are those of U^T U.
 int autotune_gram(rsg_ctx *ctx, int nb, int reps, float *best_ms, int64_t *best_kc) {
   DeviceOpGuard guard;
   if (!ctx->have_grid) return ctx->fail(RSG_ERR_STATE, "autotune_gram: grid not set");
   if (nb < 1 || reps < 1) return ctx->fail(RSG_ERR_ARG, "autotune_gram: nb and reps must be >= 1");
   const int64_t N = ctx->N;
-  double *A = nullptr, *C = nullptr;
-  if (hipMalloc(&A, size_t(N) * nb * 8) != hipSuccess) return ctx->fail(RSG_ERR_HIP, "autotune_gram: allocation failed");
+  const size_t bytes = size_t(N) * nb * 8;
+  double *A = nullptr, *B = nullptr, *C = nullptr;
+  if (hipMalloc(&A, bytes) != hipSuccess) return ctx->fail(RSG_ERR_HIP, "autotune_gram: allocation failed");
   if (hipMalloc(&C, size_t(nb) * nb * 8) != hipSuccess) {
     (void)hipFree(A);
     return ctx->fail(RSG_ERR_HIP, "autotune_gram: allocation failed");
   }
-  (void)hipMemsetAsync(A, 0x3f, size_t(N) * nb * 8, ctx->stream);
-  std::vector<int64_t> cand{0};
-  for (int c = 8; c <= 512; c *= 2)
-    if (N / c >= 512) cand.push_back((N + c - 1) / c);
-  if (gram_own(nb, true)) {
-    const int64_t kc = gram_chunk(ctx, nb, N, true);
-    if (kc > 0 && kc < N) cand.push_back(kc);
+  // a second block only where its product is timed; without room for one
+  // that product keeps its default
+  if (gram_pair_timed(nb) && hipMalloc(&B, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    B = nullptr;
   }
+  (void)hipMemsetAsync(A, 0x3f, bytes, ctx->stream);
+  if (B) (void)hipMemsetAsync(B, 0x3f, bytes, ctx->stream);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   int rc = RSG_OK;
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) rc = RSG_ERR_HIP;
-  float tbest = 0.f;
-  int64_t kbest = 0;
-  for (size_t i = 0; i < cand.size() && !rc; ++i) {
-    rc = gemm_tn_gram(ctx, nb, N, 1.0, A, A, C, cand[i]);  // warm-up (and scratch sizing)
-    if (!rc && hipEventRecord(e0, ctx->stream) != hipSuccess) rc = RSG_ERR_HIP;
-    for (int r = 0; r < reps && !rc; ++r) rc = gemm_tn_gram(ctx, nb, N, 1.0, A, A, C, cand[i]);
-    float ms = 0.f;
-    if (!rc && (hipEventRecord(e1, ctx->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-                hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
-      rc = RSG_ERR_HIP;
-    if (!rc && (i == 0 || ms < tbest)) {
-      tbest = ms;
-      kbest = cand[i];
+  // the candidates from the given one on
+  auto tune = [&](int form, const double *X, size_t from, float &tbest, int64_t &kbest) {
+    const std::vector<int64_t> cand = gram_candidates(nb, N, form);
+    for (size_t i = from; i < cand.size() && !rc; ++i) {
+      rc = gemm_tn_gram(ctx, nb, N, 1.0, A, X, C, cand[i]);  // warm-up (and scratch sizing)
+      if (!rc && hipEventRecord(e0, ctx->stream) != hipSuccess) rc = RSG_ERR_HIP;
+      for (int r = 0; r < reps && !rc; ++r) rc = gemm_tn_gram(ctx, nb, N, 1.0, A, X, C, cand[i]);
+      float ms = 0.f;
+      if (!rc && (hipEventRecord(e1, ctx->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
+                  hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
+        rc = RSG_ERR_HIP;
+      if (!rc && (i == from || ms < tbest)) {
+        tbest = ms;
+        kbest = cand[i];
+      }
     }
-  }
+  };
+  float tsame = 0.f, tpair = 0.f;
+  int64_t ksame = 0, kpair = 0;
+  tune(kGramSame, A, 0, tsame, ksame);
+  // one GEMM over all of K is the same rocBLAS call for two blocks: timed
+  // there only if it won here (36^3, 20 bands: 30 of 62 ms of tuning)
+  const size_t from = ksame == 0 ? 0 : 1;
+  if (B && gram_candidates(nb, N, kGramPair).size() > from)
+    tune(kGramPair, B, from, tpair, kpair);
+  else
+    kpair = gram_pair_timed(nb) ? gram_default(nb, N, kGramPair) : ksame;
   (void)hipStreamSynchronize(ctx->stream);
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   (void)hipFree(A);
+  if (B) (void)hipFree(B);
   (void)hipFree(C);
   if (rc) return rc == RSG_ERR_HIP ? ctx->fail(rc, "autotune_gram: timing failed") : rc;
-  bool found = false;
-  for (auto &e : ctx->gram_split)
-    if (e[0] == N && e[1] == nb) {
-      e[2] = kbest;
-      found = true;
-    }
-  if (!found) ctx->gram_split.push_back({N, int64_t(nb), kbest});
-  if (best_ms) *best_ms = tbest / reps;
-  if (best_kc) *best_kc = kbest;
+  gram_keep(ctx->gram_split, nb, N, ksame, kpair);
+  if (best_ms) *best_ms = tsame / reps;
+  if (best_kc) *best_kc = ksame;
   return RSG_OK;
 }
 

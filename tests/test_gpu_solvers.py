@@ -626,3 +626,36 @@ def test_gram_products_over_band_counts(orc, ngrid, nb):
     h = q.T @ ham.hpsi(q) * ham.dv
     want = np.linalg.eigvalsh(0.5 * (h + h.T))
     assert np.abs(ctx.subspace_diag() - want).max() < 1e-12 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("nb", [33, 100, 131])
+def test_tuned_gram_splits_give_the_same_products(orc, nb):
+    """After tuning, Gram-Schmidt, the subspace eigenvalues and those of the
+    FP32 store are as before up to summation order, where both FP64 products
+    run the library's kernel, none does, and only U^T U does.  FP64: 1e-12 of
+    the largest value; FP32 store: 16 eps(FP32) of it, the sums being FP64
+    over chunks of FP32 sums."""
+    from rsdft_develop_amd import gpu
+
+    cell = systems.silicon_supercell(1, ngrid_per_cell=24, nband=nb, displacement=0.05, seed=2)
+    ctx = gpu.Context().setup(cell, systems.model_vloc(cell))
+    u0 = systems.random_bands(cell.npoints, nb, seed=nb)
+
+    def products():
+        _load(ctx, u0)
+        ctx.gram_schmidt()
+        q = ctx.download_bands()
+        ritz = ctx.subspace_diag()
+        _load(ctx, u0)
+        ctx.gram_schmidt()
+        ctx.set_band_precision(32)
+        ritz32 = ctx.subspace_diag()
+        ctx.set_band_precision(64)
+        return q, ritz, ritz32
+
+    q0, r0, f0 = products()
+    print(f"case: tuned Gram splits, {nb} bands: {ctx.autotune_gram(nb, reps=2)}", flush=True)
+    q1, r1, f1 = products()
+    assert np.abs(q1 - q0).max() < 1e-12 * np.abs(q0).max()
+    assert np.abs(r1 - r0).max() < 1e-12 * np.abs(r0).max()
+    assert np.abs(f1 - f0).max() < 16 * np.finfo(np.float32).eps * np.abs(f0).max()
