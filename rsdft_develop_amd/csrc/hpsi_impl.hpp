@@ -1297,124 +1297,17 @@ template <typename T> int autotune_t(rsg_ctx *ctx, int nb, int reps, float *best
   }
   // deterministic non-trivial content: timing does not depend on values
   (void)hipMemsetAsync(psi, 0x3f, bytes, ctx->stream);
-  const size_t s = sizeof(T);
-  HpsiShape best = resolve_shape(shape_grid(ctx, ctx->have_nl), HpsiShape(), s, nb);
+  HpsiShape best;
   float tbest = 0.f;
-  int rc = time_shape<T>(ctx, psi, hpsi, nb, best, reps, &tbest);
-  auto consider = [&](HpsiShape cand) {
-    if (rc) return;
-    cand = resolve_shape(shape_grid(ctx, ctx->have_nl), cand, s, nb);
-    float t = 0.f;
-    int r = time_shape<T>(ctx, psi, hpsi, nb, cand, reps, &t);
-    if (r == RSG_ERR_UNSUPPORTED) return;  // shape does not fit this grid
-    if (r) {
-      rc = r;
-      return;
-    }
-    if (t < tbest) {
-      tbest = t;
-      best = cand;
-    }
-  };
-  for (int ry = 1; ry <= 2; ++ry) {
-    HpsiShape c = best;
-    c.ry = ry;
-    c.ty = 0;
-    c.zlen = 0;
-    consider(c);
-  }
-  if (std::is_same<T, float>::value) {
-    for (int ry = 1; ry <= 2; ++ry) {
-      HpsiShape c = best;
-      c.rx = 2;
-      c.ry = ry;
-      c.ty = 0;
-      c.zlen = 0;
-      consider(c);
-    }
-  }
-  if (best.rx == 2) {  // neighbouring divisors of n2
-    const int n2 = ctx->n[1];
-    int lo = 0, hi = 0;
-    for (int t = best.ty - best.ry; t > 0 && !lo; t -= best.ry)
-      if (pair_fits(ctx->n[0], n2, ctx->md, best.ry, t, s)) lo = t;
-    for (int t = best.ty + best.ry; t <= n2 && !hi; t += best.ry)
-      if (pair_fits(ctx->n[0], n2, ctx->md, best.ry, t, s)) hi = t;
-    for (int t : {lo, hi}) {
-      HpsiShape c = best;
-      c.ty = t;
-      c.zlen = 0;
-      if (t > 0) consider(c);
-    }
-  } else {
-    for (int f : {-2, -1, 1, 2}) {
-      HpsiShape c = best;
-      c.ty = best.ty + f * best.ry;
-      c.zlen = 0;
-      if (c.ty > 0) consider(c);
-    }
-  }
-  if (ctx->have_nl) {
-    for (int f : {2, 4}) {
-      HpsiShape c = best;
-      c.chunk = std::min(nb, best.chunk * f);
-      c.zlen = 0;
-      consider(c);
-    }
-    HpsiShape ch = best;
-    ch.chunk = std::max(1, best.chunk / 2);
-    ch.zlen = 0;
-    consider(ch);
-    for (int bt : {4, 8, 16, 20, 32}) {
-      HpsiShape c = best;
-      c.bt = bt;
-      consider(c);
-    }
-    if (ctx->have_ana && ctx->nl_mode != 1) {
-      HpsiShape c = best;
-      c.order = 1 - best.order;
-      consider(c);
+  int rc = search_shape(
+      shape_grid(ctx, ctx->have_nl), sizeof(T), nb,
+      [&](const HpsiShape &sh, float &ms) {
+        const int r = time_shape<T>(ctx, psi, hpsi, nb, sh, reps, &ms);
+        return r == RSG_ERR_UNSUPPORTED ? -1 : r;
+      },
       // the row tiles of a description built on the device come on first use
-      if (ensure_row_tiles(ctx) == RSG_OK) {
-        HpsiShape pj = best;
-        pj.proj = best.proj == 1 ? 0 : 1;
-        consider(pj);
-      }
-      {  // segment projections with 64 bands per wave
-        HpsiShape pj = best;
-        pj.proj = best.proj == 2 ? 0 : 2;
-        consider(pj);
-      }
-      if (best.proj != 1)  // fewer segment waves in flight per CU
-        for (int kib : {4, 8, 16, 32}) {
-          HpsiShape pl = best;
-          pl.plds = kib;
-          consider(pl);
-        }
-      if (best.proj != 1)  // segments in pieces: chords shared by two spheres read close in time
-        for (int np : {2, 4, 8}) {
-          HpsiShape ps = best;
-          ps.psplit = np;
-          consider(ps);
-        }
-      for (int f : {4, 8}) {  // smaller chunks keep psi and H psi in the Infinity Cache
-        HpsiShape d = best;
-        d.chunk = std::max(1, nb / f);
-        d.zlen = 0;
-        consider(d);
-      }
-    }
-  }
-  for (int zf : {2, 4}) {
-    HpsiShape c = best;
-    c.zlen = std::max(1, best.zlen / zf);
-    consider(c);
-  }
-  {
-    HpsiShape c = best;
-    c.zlen = ctx->n[2];
-    consider(c);
-  }
+      [&] { return ensure_row_tiles(ctx) == RSG_OK; }, best, tbest);
+  if (rc < 0) rc = RSG_ERR_UNSUPPORTED;  // not even the derived shape fits
   (void)hipStreamSynchronize(ctx->stream);
   (void)hipFree(psi);
   (void)hipFree(hpsi);

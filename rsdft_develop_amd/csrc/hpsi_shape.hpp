@@ -5,6 +5,8 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstdint>
+#include <tuple>
+#include <vector>
 
 namespace rsg {
 
@@ -274,6 +276,139 @@ inline HpsiShape resolve_shape(const HpsiGrid &gr, const HpsiShape &in, size_t s
   if (sh.proj < 0 || sh.proj > 2) sh.proj = 0;
   if (sh.plds < 0 || sh.plds > 64) sh.plds = 0;
   return sh;
+}
+
+inline std::tuple<int, int, int, int, int, int, int, int, int, int> shape_key(const HpsiShape &h) {
+  return {h.ry, h.ty, h.zlen, h.chunk, h.bt, h.order, h.rx, h.proj, h.plds, h.psplit};
+}
+
+// Coordinate search over the launch shape for nb bands of s-byte values, from
+// the derived shape on.  time(shape, ms) gives 0, or an error code that ends
+// the search, or a negative value where the shape does not fit;
+// rows_ready() makes the row tiles of the second projection form and says
+// whether there are any.  No shape is timed twice.  best and tbest receive
+// the fastest shape and its time.
+//
+// Each field's whole range is timed, also where the derived shape already
+// holds the value that is fastest on large grids: 36^3, 20 bands FP32 run
+// 32 us with one point and one row a thread, 36 with the pair kernel.
+template <typename Time, typename Rows>
+int search_shape(const HpsiGrid &gr, size_t s, int nb, Time time, Rows rows_ready, HpsiShape &best, float &tbest) {
+  const int n2 = gr.n2;
+  std::vector<HpsiShape> timed;
+  best = resolve_shape(gr, HpsiShape(), s, nb);
+  int rc = time(best, tbest);
+  if (rc) return rc;
+  timed.push_back(best);
+  auto consider = [&](const HpsiShape &in) {
+    if (rc) return;
+    const HpsiShape cand = resolve_shape(gr, in, s, nb);
+    if (cand.ty == 0) return;
+    for (const HpsiShape &h : timed)
+      if (shape_key(h) == shape_key(cand)) return;
+    timed.push_back(cand);
+    float t = 0.f;
+    const int r = time(cand, t);
+    if (r < 0) return;  // does not fit this grid
+    if (r) {
+      rc = r;
+      return;
+    }
+    if (t < tbest) {
+      tbest = t;
+      best = cand;
+    }
+  };
+  for (int rx = 1; rx <= (s == sizeof(float) ? 2 : 1); ++rx)
+    for (int ry = 1; ry <= 2; ++ry) {
+      HpsiShape c = best;
+      c.rx = rx;
+      c.ry = ry;
+      c.ty = 0;
+      c.zlen = 0;
+      consider(c);
+    }
+  if (best.rx == 2) {  // neighbouring divisors of n2
+    int lo = 0, hi = 0;
+    for (int t = best.ty - best.ry; t > 0 && !lo; t -= best.ry)
+      if (pair_fits(gr.n1, n2, gr.md, best.ry, t, s)) lo = t;
+    for (int t = best.ty + best.ry; t <= n2 && !hi; t += best.ry)
+      if (pair_fits(gr.n1, n2, gr.md, best.ry, t, s)) hi = t;
+    for (int t : {lo, hi}) {
+      HpsiShape c = best;
+      c.ty = t;
+      c.zlen = 0;
+      if (t > 0) consider(c);
+    }
+  } else {
+    for (int f : {-2, -1, 1, 2}) {
+      HpsiShape c = best;
+      c.ty = best.ty + f * best.ry;
+      c.zlen = 0;
+      if (c.ty > 0) consider(c);
+    }
+  }
+  if (gr.nonlocal) {
+    for (int f : {2, 4}) {
+      HpsiShape c = best;
+      c.chunk = std::min(nb, best.chunk * f);
+      c.zlen = 0;
+      consider(c);
+    }
+    HpsiShape ch = best;
+    ch.chunk = std::max(1, best.chunk / 2);
+    ch.zlen = 0;
+    consider(ch);
+    for (int bt : {4, 8, 16, 20, 32}) {
+      HpsiShape c = best;
+      c.bt = bt;
+      consider(c);
+    }
+    if (gr.analytic) {
+      HpsiShape c = best;
+      c.order = 1 - best.order;
+      consider(c);
+      if (rows_ready()) {
+        HpsiShape pj = best;
+        pj.proj = best.proj == 1 ? 0 : 1;
+        consider(pj);
+      }
+      {  // segment projections with 64 bands per wave
+        HpsiShape pj = best;
+        pj.proj = best.proj == 2 ? 0 : 2;
+        consider(pj);
+      }
+      if (best.proj != 1)  // fewer segment waves in flight per CU
+        for (int kib : {4, 8, 16, 32}) {
+          HpsiShape pl = best;
+          pl.plds = kib;
+          consider(pl);
+        }
+      if (best.proj != 1)  // segments in pieces: chords shared by two spheres read close in time
+        for (int np : {1, 2, 4, 8}) {
+          HpsiShape ps = best;
+          ps.psplit = np;
+          consider(ps);
+        }
+      for (int f : {4, 8}) {  // smaller chunks keep psi and H psi in the Infinity Cache
+        HpsiShape d = best;
+        d.chunk = std::max(1, nb / f);
+        d.zlen = 0;
+        consider(d);
+      }
+    }
+  }
+  for (int zf : {2, 4}) {
+    HpsiShape c = best;
+    c.zlen = std::max(1, best.zlen / zf);
+    consider(c);
+  }
+  {
+    HpsiShape c = best;
+    c.zlen = gr.n3;
+    consider(c);
+  }
+  return rc;
 }
 
 }  // namespace rsg

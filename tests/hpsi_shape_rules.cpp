@@ -3,6 +3,10 @@
 // output line.
 //   resolve n1 n2 n3 md size nb nonlocal analytic nseg  ry ty zlen chunk bt rx psplit
 //     -> ry ty zlen chunk bt rx psplit fits
+//   search n1 n2 n3 md size nb nonlocal analytic nseg  ry rx psplit chunk
+//     the autotuner's search with a clock that prefers these values (0: no
+//     preference) -> the count of timed shapes, the best shape, and each
+//     shape timed, in order: ry ty zlen chunk bt order rx proj plds psplit
 #include <cstdio>
 #include <iostream>
 #include <sstream>
@@ -25,6 +29,37 @@ HpsiGrid read_grid(std::istream &in, size_t &s, int &nb) {
   return g;
 }
 
+void print(const HpsiShape &h) {
+  std::printf(" %d %d %d %d %d %d %d %d %d %d", h.ry, h.ty, h.zlen, h.chunk, h.bt, h.order, h.rx, h.proj, h.plds,
+              h.psplit);
+}
+
+int search(std::istream &in) {
+  size_t s = 0;
+  int nb = 0;
+  const HpsiGrid g = read_grid(in, s, nb);
+  HpsiShape want, best;
+  in >> want.ry >> want.rx >> want.psplit >> want.chunk;
+  std::vector<HpsiShape> seen;
+  float t = 0.f;
+  const int rc = search_shape(
+      g, s, nb,
+      [&](const HpsiShape &h, float &ms) {
+        if (!fits(g, h, s)) return -1;
+        seen.push_back(h);
+        ms = 100.f;
+        for (auto f : {&HpsiShape::ry, &HpsiShape::rx, &HpsiShape::psplit, &HpsiShape::chunk})
+          if (want.*f && h.*f == want.*f) ms -= 10.f;
+        return 0;
+      },
+      [] { return true; }, best, t);
+  std::printf("%d", int(seen.size()));
+  print(best);
+  for (const HpsiShape &h : seen) print(h);
+  std::printf("\n");
+  return rc;
+}
+
 }  // namespace
 
 int main() {
@@ -32,6 +67,10 @@ int main() {
   while (std::getline(std::cin, line)) {
     std::istringstream in(line);
     in >> what;
+    if (what == "search") {
+      if (search(in) || !in) return 2;
+      continue;
+    }
     size_t s = 0;
     int nb = 0;
     const HpsiGrid g = read_grid(in, s, nb);

@@ -24,10 +24,11 @@ def rules(tmp_path_factory):
     subprocess.run([cxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-I", CSRC,
                     os.path.join(HERE, "hpsi_shape_rules.cpp"), "-o", exe], check=True)
 
-    def ask(lines):
+    def ask(lines, raw=False):
         r = subprocess.run([exe], input="\n".join(lines) + "\n", capture_output=True, text=True, timeout=60)
         assert r.returncode == 0, f"exit {r.returncode} after {len(r.stdout.splitlines())} of {len(lines)} answers"
-        return [dict(zip(FIELDS, map(int, a.split()))) for a in r.stdout.splitlines()]
+        rows = [list(map(int, a.split())) for a in r.stdout.splitlines()]
+        return rows if raw else [dict(zip(FIELDS, a)) for a in rows]
 
     return ask
 
@@ -85,3 +86,34 @@ def test_tile_rows_that_fit_no_kernel_are_replaced(rules):
     for size in (8, 4):
         sh, derived = rules([_resolve((72, 72, 72), size=size, ty=97), _resolve((72, 72, 72), size=size)])
         assert sh == derived and sh["fits"]
+
+
+SHAPE = ("ry", "ty", "zlen", "chunk", "bt", "order", "rx", "proj", "plds", "psplit")
+
+
+def _search(rules, n, size, nb, analytic=1, ry=0, rx=0, psplit=0, chunk=0):
+    row, = rules([f"search {n[0]} {n[1]} {n[2]} 6 {size} {nb} 1 {analytic} 2000 {ry} {rx} {psplit} {chunk}"], raw=True)
+    shapes = [dict(zip(SHAPE, row[1 + 10 * k:11 + 10 * k])) for k in range(row[0] + 1)]
+    return shapes[0], shapes[1:]
+
+
+@pytest.mark.parametrize("n,size", [((36, 36, 36), 4), ((72, 72, 72), 4), ((72, 72, 72), 8), ((108, 108, 108), 8),
+                                    ((75, 38, 70), 4), ((75, 38, 70), 8)])
+def test_autotuner_times_every_value_once(rules, n, size):
+    """One and two rows a thread, one and two points a thread where the pair
+    kernel fits, all piece counts; no shape twice, the derived one first."""
+    best, timed = _search(rules, n, size, 40)
+    derived, = rules([_resolve(n, size=size, nb=40)])
+    assert all(timed[0][k] == derived[k] for k in FIELDS[:-1]) and best == timed[0]
+    assert len({tuple(t.values()) for t in timed}) == len(timed)
+    pair = size == 4 and n[0] % 2 == 0
+    assert {(t["rx"], t["ry"]) for t in timed} == {(x, y) for x in ((1, 2) if pair else (1,)) for y in (1, 2)}
+    assert {t["psplit"] for t in timed} == {1, 2, 4, 8}
+    assert {t["bt"] for t in timed} == {4, 8, 16, 20, 32} and {t["proj"] for t in timed} == {0, 1, 2}
+
+
+@pytest.mark.parametrize("want", [dict(rx=1), dict(rx=1, ry=1), dict(rx=2, ry=1), dict(psplit=1), dict(psplit=8, rx=1),
+                                  dict(chunk=20)])
+def test_autotuner_finds_what_is_fast(rules, want):
+    best, _ = _search(rules, (72, 72, 72), 4, 160, **want)
+    assert all(best[k] == v for k, v in want.items()), best
