@@ -1098,21 +1098,26 @@ int launch_kinetic(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, int 
   return RSG_OK;
 }
 
+// Bands whose `nred` reduced and `npart` partial values a caller's scratch
+// holds (0: not one).
+template <typename T> int scratch_bands(const HpsiScratch &scr, size_t nred, size_t npart) {
+  const size_t per_band = std::max<size_t>(1, nred + npart) * sizeof(T);
+  return scr.bytes < per_band + 256 ? 0 : int(std::min<size_t>(65535, (scr.bytes - 256) / per_band));
+}
+
 // The two projection buffers of a chunk of bands: `nred` reduced and `npart`
-// partial values per band.  From the caller's scratch (the chunk shrinks
-// until both fit; RSG_ERR_ARG when one band does not) or from the
-// context's own buffers, grown on demand.
+// partial values per band.  From the caller's scratch (which the chunk was
+// chosen to fit; RSG_ERR_ARG when one band does not) or from the context's
+// own buffers, grown on demand.
 template <typename T>
-int projection_buffers(rsg_ctx *ctx, const HpsiScratch *scr, size_t nred, size_t npart, HpsiShape &sh,
+int projection_buffers(rsg_ctx *ctx, const HpsiScratch *scr, size_t nred, size_t npart, const HpsiShape &sh,
                        T **red, T **part) {
   if (scr) {
-    const size_t per_band = (nred + npart) * sizeof(T) + 256;
-    if (per_band > scr->bytes)
-      return ctx->fail(RSG_ERR_ARG, "hpsi: the projections of one band need " + std::to_string(per_band) +
+    if (sh.chunk > scratch_bands<T>(*scr, nred, npart))
+      return ctx->fail(RSG_ERR_ARG, "hpsi: the projections of one band need " +
+                                        std::to_string((nred + npart) * sizeof(T) + 256) +
                                         " bytes of scratch, more than the " + std::to_string(scr->bytes) +
                                         " available");
-    const int fit = int(std::min<size_t>(65535, (scr->bytes - 256) / ((nred + npart) * sizeof(T))));
-    if (sh.chunk > fit) sh.chunk = fit;
     const uintptr_t base = reinterpret_cast<uintptr_t>(scr->p);
     *red = reinterpret_cast<T *>(base);
     *part = reinterpret_cast<T *>((base + nred * sh.chunk * sizeof(T) + 255) & ~uintptr_t(255));
@@ -1133,20 +1138,35 @@ int launch_hpsi(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, const H
   if (nb == 0) return RSG_OK;
   if (nb > 65535) return ctx->fail(RSG_ERR_ARG, "hpsi: nb above 65535");
   if (!psi || !hpsi) return ctx->fail(RSG_ERR_ARG, "hpsi: null buffer");
-  HpsiShape sh = resolve_shape(shape_grid(ctx, ctx->have_nl), shape_of<T>(ctx), sizeof(T), nb);
+  HpsiGrid gr = shape_grid(ctx, ctx->have_nl);
+  const HpsiShape &asked = shape_of<T>(ctx);
+  // values per band of the analytic form's two projection buffers
+  bool rows = false;
+  int npc = 1;  // partial slots per segment
+  size_t nred = 0, npart = 0;
+  if (gr.analytic) {
+    AnalyticDev<T> &an = ana_of<T>(ctx);
+    rows = asked.proj == 1 && row_tiles_fit<T>(ctx, an);
+    nred = size_t(an.ngroup) * 4;
+    if (!rows) npc = asked.psplit ? asked.psplit : kAutoPieces;
+    const auto part = [&] { return size_t(rows ? an.rt_nslot : an.nseg * npc) * 4; };
+    if (scr && asked.psplit == 0)  // a caller's scratch takes fewer pieces before it refuses a band
+      while (npc > 1 && (nred + part()) * sizeof(T) + 256 > scr->bytes) npc /= 2;
+    npart = part();
+  } else if (gr.nonlocal) {
+    nred = size_t(ctx->tables.nzlma);
+    npart = size_t(nl_of<T>(ctx).nseg) * 4;
+  }
+  if (scr && gr.nonlocal) gr.max_chunk = scratch_bands<T>(*scr, nred, npart);
+  HpsiShape sh = resolve_shape(gr, asked, sizeof(T), nb);
   if (sh.ty == 0) return no_stencil_tile(ctx);
   if (!ctx->have_nl) {
     int rc = launch_stencil<T>(ctx, psi, hpsi, ld, nb, sh, 0);
     if (rc) return rc;
-  } else if (ctx->nl_mode != 1 && ctx->have_ana) {
+  } else if (gr.analytic) {
     AnalyticDev<T> &an = ana_of<T>(ctx);
     T *cp = nullptr, *part = nullptr;
-    const bool rows = sh.proj == 1 && row_tiles_fit<T>(ctx, an);
-    int npc = rows ? 1 : sh.psplit;  // partial slots per segment
-    if (scr && shape_of<T>(ctx).psplit == 0)  // a caller's scratch takes fewer pieces before it refuses a band
-      while (npc > 1 && size_t(4) * (size_t(an.ngroup) + size_t(an.nseg) * npc) * sizeof(T) + 256 > scr->bytes) npc /= 2;
-    const int npart = rows ? an.rt_nslot : an.nseg * npc;
-    int rc0 = projection_buffers<T>(ctx, scr, size_t(an.ngroup) * 4, size_t(npart) * 4, sh, &cp, &part);
+    int rc0 = projection_buffers<T>(ctx, scr, nred, npart, sh, &cp, &part);
     if (rc0) return rc0;
     for (int c0 = 0; c0 < nb; c0 += sh.chunk) {
       const int nbc = std::min(sh.chunk, nb - c0);
@@ -1204,7 +1224,7 @@ int launch_hpsi(rsg_ctx *ctx, const T *psi, T *hpsi, int64_t ld, int nb, const H
     constexpr int BB = 8;
     T *uv = nullptr, *part = nullptr;
     if (scr) {
-      int rc0 = projection_buffers<T>(ctx, scr, size_t(nz), size_t(nl.nseg) * 4, sh, &uv, &part);
+      int rc0 = projection_buffers<T>(ctx, scr, nred, npart, sh, &uv, &part);
       if (rc0) return rc0;
     } else {
       if (ctx->uvunk.ensure(size_t(nz) * sh.chunk * sizeof(T)) != hipSuccess ||

@@ -34,6 +34,7 @@ struct HpsiGrid {
   bool nonlocal = false;  // a nonlocal part runs beside the stencil
   bool analytic = false;  // ... in the analytic form
   int nseg = 0;           // sphere segments of the analytic form
+  int max_chunk = 0;      // bands whose projections a caller's scratch holds, 0 = any number
 };
 
 constexpr size_t kMaxDynLds = 64 * 1024;
@@ -235,6 +236,10 @@ inline HpsiShape resolve_shape(const HpsiGrid &gr, const HpsiShape &in, size_t s
     }
   }
   sh.chunk = std::max(1, std::min(sh.chunk, nb));
+  if (gr.max_chunk > 0 && sh.chunk > gr.max_chunk) {  // before z-runs and apply waves, which follow from it
+    const int nch = (nb + gr.max_chunk - 1) / gr.max_chunk;
+    sh.chunk = (nb + nch - 1) / nch;
+  }
   if (sh.zlen <= 0) {
     int tiles = (n2 + sh.ty - 1) / sh.ty, waves, per_cu;
     if (sh.rx == 2) {
@@ -291,7 +296,7 @@ inline std::tuple<int, int, int, int, int, int, int, int, int, int> shape_key(co
 //
 // Each field's whole range is timed, also where the derived shape already
 // holds the value that is fastest on large grids: 36^3, 20 bands FP32 run
-// 32 us with one point and one row a thread, 36 with the pair kernel.
+// 28 us with one point and one row a thread, 37 with the pair kernel.
 template <typename Time, typename Rows>
 int search_shape(const HpsiGrid &gr, size_t s, int nb, Time time, Rows rows_ready, HpsiShape &best, float &tbest) {
   const int n2 = gr.n2;

@@ -1,7 +1,7 @@
 // The launch-shape rules of csrc/hpsi_shape.hpp behind a line protocol, for
 // tests/test_hpsi_shape_rules.py: one request per input line, one answer per
 // output line.
-//   resolve n1 n2 n3 md size nb nonlocal analytic nseg  ry ty zlen chunk bt rx psplit
+//   resolve n1 n2 n3 md size nb nonlocal analytic nseg  ry ty zlen chunk bt rx psplit max_chunk
 //     -> ry ty zlen chunk bt rx psplit fits
 //   search n1 n2 n3 md size nb nonlocal analytic nseg  ry rx psplit chunk
 //     the autotuner's search with a clock that prefers these values (0: no
@@ -73,9 +73,9 @@ int main() {
     }
     size_t s = 0;
     int nb = 0;
-    const HpsiGrid g = read_grid(in, s, nb);
+    HpsiGrid g = read_grid(in, s, nb);
     HpsiShape a;
-    in >> a.ry >> a.ty >> a.zlen >> a.chunk >> a.bt >> a.rx >> a.psplit;
+    in >> a.ry >> a.ty >> a.zlen >> a.chunk >> a.bt >> a.rx >> a.psplit >> g.max_chunk;
     if (!in || what != "resolve") return 2;
     const HpsiShape sh = resolve_shape(g, a, s, nb);
     std::printf("%d %d %d %d %d %d %d %d\n", sh.ry, sh.ty, sh.zlen, sh.chunk, sh.bt, sh.rx, sh.psplit,

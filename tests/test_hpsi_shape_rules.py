@@ -33,10 +33,10 @@ def rules(tmp_path_factory):
     return ask
 
 
-def _resolve(n, md=6, size=8, nb=64, nonlocal_=1, analytic=1, nseg=2000, **shape):
+def _resolve(n, md=6, size=8, nb=64, nonlocal_=1, analytic=1, nseg=2000, max_chunk=0, **shape):
     s = {k: shape.get(k, 0) for k in FIELDS[:-1]}
     return (f"resolve {n[0]} {n[1]} {n[2]} {md} {size} {nb} {nonlocal_} {analytic} {nseg} "
-            f"{s['ry']} {s['ty']} {s['zlen']} {s['chunk']} {s['bt']} {s['rx']} {s['psplit']}")
+            f"{s['ry']} {s['ty']} {s['zlen']} {s['chunk']} {s['bt']} {s['rx']} {s['psplit']} {max_chunk}")
 
 
 @pytest.mark.parametrize("size", [8, 4])
@@ -117,3 +117,17 @@ def test_autotuner_times_every_value_once(rules, n, size):
 def test_autotuner_finds_what_is_fast(rules, want):
     best, _ = _search(rules, (72, 72, 72), 4, 160, **want)
     assert all(best[k] == v for k, v in want.items()), best
+
+
+@pytest.mark.parametrize("n,nb", [((72, 72, 72), 160), ((108, 108, 108), 480), ((144, 144, 144), 1100)])
+@pytest.mark.parametrize("limit", [1, 10, 37, 5000])
+@pytest.mark.parametrize("analytic", [0, 1])
+def test_z_runs_and_apply_waves_suit_the_chunk_a_scratch_holds(rules, n, nb, limit, analytic):
+    """A caller's scratch bounds the bands of a chunk: the shape is the one
+    for chunks of that many bands, in chunks of equal size."""
+    free, sh = rules([_resolve(n, nb=nb, analytic=analytic), _resolve(n, nb=nb, analytic=analytic, max_chunk=limit)])
+    assert sh["chunk"] <= limit and -(-nb // sh["chunk"]) == -(-nb // min(limit, free["chunk"]))
+    same, = rules([_resolve(n, nb=nb, analytic=analytic, chunk=sh["chunk"])])
+    assert sh == same
+    given, = rules([_resolve(n, nb=nb, analytic=analytic, chunk=7, zlen=5, bt=8, max_chunk=limit)])
+    assert (given["zlen"], given["bt"], given["chunk"] <= min(7, limit)) == (5, 8, True)
