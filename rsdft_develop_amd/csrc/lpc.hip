@@ -292,22 +292,23 @@ __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ tgt, con
 template <int C>
 __global__ __launch_bounds__(256) void k_quads(const uint16_t *__restrict__ in, int64_t nrow, int n1, int nq, int wrap,
                                                uint16_t *__restrict__ out) {
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= nrow * nq * C) return;
-  const int c = int(t % C), q = int((t / C) % nq);
-  const int64_t row = t / (int64_t(C) * nq);
-  uint16_t v[4];
+  for (int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < nrow * nq * C;
+       t += int64_t(gridDim.x) * blockDim.x) {
+    const int c = int(t % C), q = int((t / C) % nq);
+    const int64_t row = t / (int64_t(C) * nq);
+    uint16_t v[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int x = 4 * (q - 1) + i;
-    if (wrap && x == -1) x = n1 - 1;
-    else if (wrap && x == n1) x = 0;
-    v[i] = x >= 0 && x < n1 ? in[(row * n1 + x) * C + c] : uint16_t(0);
+    for (int i = 0; i < 4; ++i) {
+      int x = 4 * (q - 1) + i;
+      if (wrap && x == -1) x = n1 - 1;
+      else if (wrap && x == n1) x = 0;
+      v[i] = x >= 0 && x < n1 ? in[(row * n1 + x) * C + c] : uint16_t(0);
+    }
+    uint2 w;
+    w.x = uint32_t(v[0]) | (uint32_t(v[1]) << 16);
+    w.y = uint32_t(v[2]) | (uint32_t(v[3]) << 16);
+    *reinterpret_cast<uint2 *>(out + 4 * t) = w;
   }
-  uint2 w;
-  w.x = uint32_t(v[0]) | (uint32_t(v[1]) << 16);
-  w.y = uint32_t(v[2]) | (uint32_t(v[3]) << 16);
-  *reinterpret_cast<uint2 *>(out + 4 * t) = w;
 }
 
 // dW[co][k] += sum_p dz[p][co] X[k][p], k = tap * CIN + ci, on MFMA with
@@ -622,34 +623,53 @@ int forward_t(rsg_ctx *ctx, const T *g, int64_t ldg, int nsamp, T *pg, bool trai
 // quads of a line: one in front, the 16-point chunks, one behind
 int quads_per_line(const rsg_ctx *ctx) { return 4 * ((ctx->n[0] + 15) / 16) + 2; }
 
+// Samples whose quad layouts are held at once: both buffers, at the 16
+// channels that each holds at some layer, within 1 GiB; at least one sample.
+// The layout takes 1.6 times the field for 36 points a line, 2.4 times for
+// 17; a batch of 16 samples of 36^3 points takes 74 MB.
+constexpr int64_t kQuadBytes = int64_t(1) << 30;
+int quad_samples(const rsg_ctx *ctx, int nsamp) {
+  const int64_t per = int64_t(ctx->n[1]) * ctx->n[2] * quads_per_line(ctx) * 2 * 16 * 8;
+  return int(std::max<int64_t>(1, std::min<int64_t>(nsamp, kQuadBytes / per)));
+}
+
 template <int C> void to_quads(rsg_ctx *ctx, int nsamp, const uint16_t *in, int wrap, uint16_t *out) {
   const int64_t nrow = int64_t(ctx->n[1]) * ctx->n[2] * nsamp;
   const int nq = quads_per_line(ctx);
   const int64_t n = nrow * nq * C;
-  hipLaunchKernelGGL((k_quads<C>), dim3(unsigned((n + 255) / 256)), dim3(256), 0, ctx->stream, in, nrow, ctx->n[0], nq,
-                     wrap, out);
+  // a launch holds fewer than 2^32 threads
+  const unsigned nblk = unsigned(std::min<int64_t>((n + 255) / 256, int64_t(1) << 23));
+  hipLaunchKernelGGL((k_quads<C>), dim3(nblk), dim3(256), 0, ctx->stream, in, nrow, ctx->n[0], nq, wrap, out);
 }
 
-// gradient of a layer's weights into out and of its biases into db
+// gradient of a layer's weights into out and of its biases into db; the
+// samples go through the quad buffers in groups, whose partial sums lie one
+// after another
 template <int CIN, int KP, int COUT>
 int weight_grad(rsg_ctx *ctx, int nsamp, const uint16_t *in, const uint16_t *dz, float *out, float *db) {
   LpcState &L = ctx->lpc;
   const Grid3 g{ctx->n[0], ctx->n[1], ctx->n[2]};
-  const int64_t nrow = int64_t(g.n2) * g.n3 * nsamp, total = ctx->N * nsamp;
-  const int nq = quads_per_line(ctx);
-  if (nrow > 0x7fffffff) return ctx->fail(RSG_ERR_UNSUPPORTED, "lpc: too many lines");
-  const int nblk = int(std::min<int64_t>(512, (nrow + 15) / 16));
+  const int64_t N = ctx->N, n23 = int64_t(g.n2) * g.n3, total = N * nsamp;
+  const int nq = quads_per_line(ctx), per = quad_samples(ctx, nsamp);
+  auto blocks = [&](int ns) { return int(std::min<int64_t>(512, (n23 * ns + 15) / 16)); };
+  const int64_t nblk = int64_t(nsamp / per) * blocks(per) + (nsamp % per ? blocks(nsamp % per) : 0);
   const unsigned nbb = unsigned(std::min<int64_t>(512, (total * COUT + 8 * 256 - 1) / (8 * 256)));
   if (L.part.ensure(std::max(size_t(nblk) * 16 * KP, size_t(nbb) * COUT) * 4) != hipSuccess ||
-      L.xq.ensure(size_t(nrow) * nq * CIN * 8) != hipSuccess || L.dq.ensure(size_t(nrow) * nq * COUT * 8) != hipSuccess)
+      L.xq.ensure(size_t(n23) * per * nq * CIN * 8) != hipSuccess ||
+      L.dq.ensure(size_t(n23) * per * nq * COUT * 8) != hipSuccess)
     return ctx->fail(RSG_ERR_HIP, "lpc: allocation failed");
   float *part = L.part.as<float>();
-  to_quads<CIN>(ctx, nsamp, in, 1, L.xq.as<uint16_t>());
-  to_quads<COUT>(ctx, nsamp, dz, 0, L.dq.as<uint16_t>());
-  hipLaunchKernelGGL((k_conv_dw<CIN, KP, COUT>), dim3(nblk), dim3(256), 0, ctx->stream, g, nsamp, L.xq.as<uint16_t>(),
-                     L.dq.as<uint16_t>(), nq, part);
+  int64_t b0 = 0;
+  for (int s0 = 0; s0 < nsamp; s0 += per) {
+    const int ns = std::min(per, nsamp - s0), nb = blocks(ns);
+    to_quads<CIN>(ctx, ns, in + int64_t(s0) * N * CIN, 1, L.xq.as<uint16_t>());
+    to_quads<COUT>(ctx, ns, dz + int64_t(s0) * N * COUT, 0, L.dq.as<uint16_t>());
+    hipLaunchKernelGGL((k_conv_dw<CIN, KP, COUT>), dim3(nb), dim3(256), 0, ctx->stream, g, ns, L.xq.as<uint16_t>(),
+                       L.dq.as<uint16_t>(), nq, part + b0 * 16 * KP);
+    b0 += nb;
+  }
   const int len = 16 * KP;
-  hipLaunchKernelGGL(k_sum_parts, dim3((len + 63) / 64), dim3(1024), 0, ctx->stream, part, nblk, len, out);
+  hipLaunchKernelGGL(k_sum_parts, dim3((len + 63) / 64), dim3(1024), 0, ctx->stream, part, int(nblk), len, out);
   hipLaunchKernelGGL(k_bias_grad<COUT>, dim3(nbb), dim3(256), 0, ctx->stream, dz, total, part);
   hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(1024), 0, ctx->stream, part, int(nbb), COUT, db);
   return RSG_OK;

@@ -282,3 +282,53 @@ def test_trained_network_gain_over_no_preconditioner():
     assert ev["rounds_hprsdft"] == 8
     assert ev["reached_learned"] and ev["reached_none"]
     assert ev["rounds_learned"] < ev["rounds_none"]
+
+
+def test_training_memory_of_a_large_batch(setup):
+    """The quad layouts of the weight gradients stay within 1 GiB, whatever
+    the batch: 648 samples of (17, 36, 36) would take 2.0 GiB.  They go
+    through in groups (323, 323 and 2 samples); loss and gradients are the
+    means over eight batches that need no groups.  Eight being a power of
+    two, every dy and dz of the whole batch is the part's exactly, so only
+    the order of the FP32 sums differs: chains of at most 409 additions,
+    1.2e-6 of a chain's terms, 3e-8 of the sum of all terms over 2048
+    chains; 1e-3 of the gradient leaves room for cancellation of 3e4."""
+    import ctypes
+
+    from rsdft_develop_amd import gpu, hip
+
+    _, p, _, rng = setup
+    n = (17, 36, 36)
+    N, ns, parts = int(np.prod(n)), 648, 8
+    ctx = gpu.Context()
+    ctx.set_grid(n, np.diag([5.1, 10.8, 10.8]), 6)
+    ctx.lpc_set_potential(0.3 * np.sin(np.arange(N) * 0.01))
+    ctx.lpc_set_params(p)
+    g = rng.standard_normal((N, ns), dtype=np.float32)
+    t = np.float32(0.5) * g + np.float32(0.2)
+    dg, dt = hip.DeviceArray.from_numpy(g), hip.DeviceArray.from_numpy(t)
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.runtime().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    print(f"case: {ns} training samples of {n}", flush=True)
+    before = free()
+    loss, grads = ctx.lpc_train_step(dg.ptr, dt.ptr, ns, want_grads=True)
+    used = before - free()
+    fields = N * ns * (4 + 32 + 32 + 4 + 2 + 32 + 32)  # two inputs, activations, y, dy, dz
+    assert used < fields + 1.25 * 2 ** 30, (used, fields)
+    step, losses, mean = ns // parts, [], 0.0
+    for k in range(parts):
+        o = k * step * N * 4
+        lk, gk = ctx.lpc_train_step(dg.ptr + o, dt.ptr + o, step, want_grads=True)
+        losses.append(lk)
+        mean = mean + gk.astype(np.float64) / parts
+    assert loss == pytest.approx(np.mean(losses), rel=1e-9)
+    for k, want in lpc.unpack(mean).items():
+        got = lpc.unpack(grads)[k]
+        assert np.linalg.norm(got - want) < 1e-3 * np.linalg.norm(want), k
+    dg.free()
+    dt.free()
+    ctx.close()
