@@ -160,17 +160,19 @@ __global__ __launch_bounds__(64 * kWaves) void k_conv(Grid3 g, int64_t N, int zl
     }
   };
   if constexpr (CIN == 16) {
-    int ofs[9];
+    // points of the plane; the channel factor goes into the 64-bit address
+    // (a plane of 2^27 points passes 2^31 channels)
+    unsigned ofs[9];
 #pragma unroll
-    for (int t = 0; t < 9; ++t) ofs[t] = (tap_wrap(x, t % 3, g.n1) + g.n1 * tap_wrap(y, t / 3, g.n2)) * 16 + 4 * lq;
+    for (int t = 0; t < 9; ++t) ofs[t] = unsigned(tap_wrap(x, t % 3, g.n1) + g.n1 * tap_wrap(y, t / 3, g.n2));
     const int64_t pstr = int64_t(n12) * 16;
     f32x4 acc[3][3];  // [output plane mod 3][chain]
     uint2 nf[9];
     int zn = z0 == 0 ? g.n3 - 1 : z0 - 1;  // input plane to fetch
     auto fetch = [&]() {
-      const uint16_t *sp = src + zn * pstr;
+      const uint16_t *sp = src + zn * pstr + 4 * lq;
 #pragma unroll
-      for (int t = 0; t < 9; ++t) nf[t] = *reinterpret_cast<const uint2 *>(sp + ofs[t]);
+      for (int t = 0; t < 9; ++t) nf[t] = *reinterpret_cast<const uint2 *>(sp + size_t(ofs[t]) * 16);
       zn = zn + 1 == g.n3 ? 0 : zn + 1;
     };
     fetch();
@@ -206,12 +208,13 @@ __global__ __launch_bounds__(64 * kWaves) void k_conv(Grid3 g, int64_t N, int zl
     // K slot k = 16 c + 4 lq + i is channel k % CIN of tap k / CIN: the
     // lane's taps, their in-plane offsets and planes
     constexpr int NT = NC * 4 / CIN;
-    int ofs[NT], dz[NT];
+    unsigned ofs[NT];
+    int dz[NT];
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
       const int t = (16 * (u / (4 / CIN)) + 4 * lq) / CIN + u % (4 / CIN), tc = min(t, 26);
       dz[u] = t < 27 ? tc / 9 : 3;  // 3: no tap
-      ofs[u] = (tap_wrap(x, tc % 3, g.n1) + g.n1 * tap_wrap(y, (tc / 3) % 3, g.n2)) * CIN;
+      ofs[u] = unsigned(tap_wrap(x, tc % 3, g.n1) + g.n1 * tap_wrap(y, (tc / 3) % 3, g.n2));
     }
     const int64_t pstr = int64_t(n12) * CIN;
     for (int z = z0; z < z1; ++z) {
@@ -220,7 +223,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_conv(Grid3 g, int64_t N, int zl
       uint32_t w[NT];
 #pragma unroll
       for (int u = 0; u < NT; ++u) {
-        const uint16_t *p = (dz[u] == 0 ? s0 : (dz[u] == 2 ? s2 : s1)) + ofs[u];
+        const uint16_t *p = (dz[u] == 0 ? s0 : (dz[u] == 2 ? s2 : s1)) + size_t(ofs[u]) * CIN;
         if constexpr (CIN == 2)
           w[u] = *reinterpret_cast<const uint32_t *>(p);
         else

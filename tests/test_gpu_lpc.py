@@ -332,3 +332,33 @@ def test_training_memory_of_a_large_batch(setup):
     dg.free()
     dt.free()
     ctx.close()
+
+
+def test_planes_beyond_two_to_the_27_points(setup):
+    """Sixteen channels of such a plane pass 2^31 values.  Input and potential
+    of +-1 repeat every five rows, so that every norm is exact and the output
+    repeats to the last bit: it is that of the five-row grid."""
+    from rsdft_develop_amd import gpu, hip
+
+    _, p, _, rng = setup
+    rows = 5 * 52429
+    assert 512 * rows > 2 ** 27
+    sign = rng.permutation(np.repeat([-1.0, 1.0], 512 * 5 // 2)), rng.permutation(np.repeat([-1.0, 1.0], 512 * 5 // 2))
+    out = []
+    for n2 in (5, rows):
+        N = 512 * n2
+        ctx = gpu.Context()
+        ctx.set_grid((512, n2, 1), np.diag([150.0, 0.3 * n2, 10.0]), 6)
+        ctx.lpc_set_potential(np.tile(sign[0], n2 // 5))
+        ctx.lpc_set_params(p)
+        d = hip.DeviceArray.from_numpy(np.tile(sign[1].astype(np.float32), n2 // 5))
+        o = hip.DeviceArray((N,), dtype=np.float32)
+        print(f"case: network on a plane of {N} points", flush=True)
+        ctx.lpc_apply_device(d.ptr, o.ptr, N, 1, dtype=np.float32)
+        ctx.synchronize()
+        out.append(o.to_numpy())
+        d.free()
+        o.free()
+        ctx.close()
+    assert np.abs(out[0]).max() > 0
+    np.testing.assert_array_equal(out[1].reshape(-1, 512 * 5), np.broadcast_to(out[0], (rows // 5, 512 * 5)))
