@@ -659,3 +659,35 @@ def test_tuned_gram_splits_give_the_same_products(orc, nb):
     assert np.abs(q1 - q0).max() < 1e-12 * np.abs(q0).max()
     assert np.abs(r1 - r0).max() < 1e-12 * np.abs(r0).max()
     assert np.abs(f1 - f0).max() < 16 * np.finfo(np.float32).eps * np.abs(f0).max()
+
+
+@pytest.mark.parametrize("ngrid,mloop", [((4, 6, 10), 4), ((20, 9, 8), 5), ((36, 36, 36), 4), ((75, 14, 11), 4),
+                                          ((144, 6, 6), 6), ((131, 9, 6), 3), ((171, 6, 5), 2), ((30, 20, 10), 1)])
+def test_precond_hprsdft_streaming_passes(orc, ngrid, mloop):
+    """The passes that sweep the grid once per CG update: four and more
+    steps, one step, and two or three on rows too long for the recomputing
+    ones; vector and one-point forms (even and odd leading dimensions), rows
+    within and beyond one wave, a zero band.  Rounding grows with the steps:
+    twice the tolerances of three steps, FP64 2e-12 and FP32 1e-4 of each
+    band's largest value."""
+    import dataclasses
+
+    from rsdft_develop_amd import gpu
+
+    cell = dataclasses.replace(systems.silicon_supercell(1, nband=4), ngrid=ngrid)
+    ham = orc.Ham(cell, vloc=None, projectors=False)
+    ctx = gpu.Context()
+    ctx.set_grid(cell.ngrid, cell.aa, cell.md)
+    N = cell.npoints
+    g = np.random.default_rng(sum(ngrid)).standard_normal((N, 4))
+    g[:, 1] *= 1e-3
+    g[:, 3] = 0.0
+    want = ham.precond(g, mloop=mloop)
+    for ld in (N + (-N) % 4, N + (-N) % 4 + 1):
+        for dt, rel in ((np.float64, 2e-12), (np.float32, 1e-4)):
+            print(f"case: precond grid {ngrid} mloop {mloop} ld N+{ld - N} {np.dtype(dt).name}", flush=True)
+            got = _precond_gpu(ctx, g, ld, mloop, dt)
+            assert not got[:, 3].any()
+            for b in range(3):
+                err = np.abs(got[:, b] - want[:, b]).max() / np.abs(want[:, b]).max()
+                assert err <= rel, (ngrid, ld - N, b, err)
