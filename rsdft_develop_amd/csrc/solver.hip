@@ -427,11 +427,6 @@ __global__ void k_cggs_mask(double *__restrict__ C, int mb, int nn, int n0, int 
   if (!keep) C[m + int64_t(mb) * j] = 0.0;
 }
 
-__global__ void k_scale_copy(const double *__restrict__ a, double s, double *__restrict__ b, int n) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) b[t] = s * a[t];
-}
-
 __global__ void k_fill(double *__restrict__ a, double v, int n) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) a[t] = v;
