@@ -145,12 +145,23 @@ inline int pick_ty_pair(int n1, int n2, int md, int ry, size_t s) {
 //   bands, two halo elements: 604 with two, 660 with one); there the rows go
 //   in parts where n1 is even (k_stencil's figures), and full rows stay for
 //   an odd n1, whose parts start misaligned (99^3, 240 bands: 3782 with full
-//   rows, 4001 with parts; 111 x 107 x 101: 4638 and 4762).  More than 1.3
-//   padded rows cost more than the second row a thread gives (75 x 38 x 70,
-//   77 bands, 1.26: 252 with two, 258 with one);
+//   rows, 4001 with parts; 111 x 107 x 101: 4638 and 4762).  Parts of 16 and
+//   more rows pay while they pad few of them: up to 1.4 padded rows (96 x 23
+//   x 60, 226 bands, 1.39: 917 in parts, 958 with one row; 108 x 13 x 72, 296
+//   bands, 1.23: 924 and 972), not above (108 x 22 x 72, 175 bands, 1.45: 929
+//   and 888; 144 x 9 x 72, 321 bands, 1.78: 1212 and 1119).  Full rows, two a
+//   thread, pad up to 1.3 (75 x 38 x 70, 150 bands, 1.26: 424 with two, 447
+//   with one); above, one row a thread where its tile stages no more than two
+//   halo elements a thread (78 x 27 x 60, 100 and 250 bands, 1.33: 203 and
+//   386 with one, 231 and 397 with two, 250 and 445 in parts; 72 x 18 x 72,
+//   100 bands: 307, 361, 401), else still two (84 x 25 x 60, 250 bands, 1.44:
+//   847 with two, 919 with one, 943 in parts);
 //   a call of few points is a chain of latencies, shorter with one row a
-//   thread (24^3, 12 bands: 27.0 with two, 24.7 with one; 36^3, 20 bands
-//   38.2 and 35.3; 40^3, 27 bands 45 either way);
+//   thread: the line at 2^20 points times bands lies where the two cross or
+//   are level on most grids (36^3, 20 bands 30.9 with one row, 33.6 with two,
+//   48 bands 52.1 and 53.3; 40^3, 12 bands 30.8 and 31.3, 40 bands 55.8 and
+//   51.4; 72^3, 1 band 56.2 and 58.5, 10 bands 81.4 and 78.6; 48^3 is an
+//   exception, 9 bands 36.2 and 32.4);
 // - FP32 takes the pair kernel where it fits (72^3, 160 bands: 330 against
 //   395; 108^3, 480 bands: 3800 against 4400);
 // - the analytic form runs all bands at once (72^3, 160 bands FP64 in
@@ -200,10 +211,13 @@ inline HpsiShape resolve_shape(const HpsiGrid &gr, const HpsiShape &in, size_t s
       const bool slow = ty == 0 || (rt.nx == 1 && rt.halo > 2 * rt.threads);  // full rows whose halo spills
       if (one) {
         if ((slow || gr.N * int64_t(nb) < kSmallCall) && one_fits(1)) sh.ry = 1;
-      } else if (slow || (n2 + ty - 1) / ty * ty > 1.3 * n2) {
+      } else if (slow) {
         const int part = ty && n1 % 2 == 0 ? pick_ty_parts(n1, n2, gr.md, s) : 0;
-        if (part) sh.ty = part;
+        if (part && (n2 + part - 1) / part * part <= 1.4 * n2) sh.ty = part;
         else sh.ry = 1;
+      } else if ((n2 + ty - 1) / ty * ty > 1.3 * n2) {
+        const RowTile r1 = row_tile(n1, gr.md, 1, pick_ty(n1, n2, gr.md, 1, s), s);
+        if (r1.fits && r1.halo <= 2 * r1.threads) sh.ry = 1;
       } else if (gr.N * int64_t(nb) < kSmallCall) {
         sh.ry = 1;
       }

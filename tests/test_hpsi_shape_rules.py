@@ -131,3 +131,17 @@ def test_z_runs_and_apply_waves_suit_the_chunk_a_scratch_holds(rules, n, nb, lim
     assert sh == same
     given, = rules([_resolve(n, nb=nb, analytic=analytic, chunk=7, zlen=5, bt=8, max_chunk=limit)])
     assert (given["zlen"], given["bt"], given["chunk"] <= min(7, limit)) == (5, 8, True)
+
+
+@pytest.mark.parametrize("n,rows", [
+    ((72, 18, 72), 1), ((80, 17, 40), 1), ((84, 16, 84), 1), ((78, 27, 60), 1),  # two full rows pad too much
+    ((84, 25, 60), 2), ((74, 25, 60), 2),                                        # ... and one row's halo spills
+    ((144, 9, 72), 1), ((108, 22, 72), 1), ((72, 9, 72), 1),                     # parts would pad too much
+    ((96, 23, 60), "parts"), ((108, 13, 72), "parts"), ((108, 108, 108), "parts"), ((144, 144, 144), "parts"),
+    ((72, 72, 72), 2), ((75, 38, 70), 2), ((99, 99, 99), 1),                     # little padding; odd rows
+])
+def test_rows_a_thread_where_tiles_pad(rules, n, rows):
+    """FP64, each choice being the faster one where they were measured."""
+    sh, = rules([_resolve(n, nb=300)])
+    parts = n[0] * sh["ty"] // sh["ry"] > 512
+    assert sh["fits"] and ("parts" if parts else sh["ry"]) == rows, sh
