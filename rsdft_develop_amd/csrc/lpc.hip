@@ -295,23 +295,22 @@ __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ tgt, con
 template <int C>
 __global__ __launch_bounds__(256) void k_quads(const uint16_t *__restrict__ in, int64_t nrow, int n1, int nq, int wrap,
                                                uint16_t *__restrict__ out) {
-  for (int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < nrow * nq * C;
-       t += int64_t(gridDim.x) * blockDim.x) {
-    const int c = int(t % C), q = int((t / C) % nq);
-    const int64_t row = t / (int64_t(C) * nq);
-    uint16_t v[4];
+  const int64_t t = (int64_t(blockIdx.y) * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t >= nrow * nq * C) return;
+  const int c = int(t % C), q = int((t / C) % nq);
+  const int64_t row = t / (int64_t(C) * nq);
+  uint16_t v[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int x = 4 * (q - 1) + i;
-      if (wrap && x == -1) x = n1 - 1;
-      else if (wrap && x == n1) x = 0;
-      v[i] = x >= 0 && x < n1 ? in[(row * n1 + x) * C + c] : uint16_t(0);
-    }
-    uint2 w;
-    w.x = uint32_t(v[0]) | (uint32_t(v[1]) << 16);
-    w.y = uint32_t(v[2]) | (uint32_t(v[3]) << 16);
-    *reinterpret_cast<uint2 *>(out + 4 * t) = w;
+  for (int i = 0; i < 4; ++i) {
+    int x = 4 * (q - 1) + i;
+    if (wrap && x == -1) x = n1 - 1;
+    else if (wrap && x == n1) x = 0;
+    v[i] = x >= 0 && x < n1 ? in[(row * n1 + x) * C + c] : uint16_t(0);
   }
+  uint2 w;
+  w.x = uint32_t(v[0]) | (uint32_t(v[1]) << 16);
+  w.y = uint32_t(v[2]) | (uint32_t(v[3]) << 16);
+  *reinterpret_cast<uint2 *>(out + 4 * t) = w;
 }
 
 // dW[co][k] += sum_p dz[p][co] X[k][p], k = tap * CIN + ci, on MFMA with
@@ -639,10 +638,10 @@ int quad_samples(const rsg_ctx *ctx, int nsamp) {
 template <int C> void to_quads(rsg_ctx *ctx, int nsamp, const uint16_t *in, int wrap, uint16_t *out) {
   const int64_t nrow = int64_t(ctx->n[1]) * ctx->n[2] * nsamp;
   const int nq = quads_per_line(ctx);
-  const int64_t n = nrow * nq * C;
-  // a launch holds fewer than 2^32 threads
-  const unsigned nblk = unsigned(std::min<int64_t>((n + 255) / 256, int64_t(1) << 23));
-  hipLaunchKernelGGL((k_quads<C>), dim3(nblk), dim3(256), 0, ctx->stream, in, nrow, ctx->n[0], nq, wrap, out);
+  // a launch holds fewer than 2^32 threads in a dimension
+  const int64_t nblk = (nrow * nq * C + 255) / 256, gx = std::min<int64_t>(nblk, int64_t(1) << 23);
+  hipLaunchKernelGGL((k_quads<C>), dim3(unsigned(gx), unsigned((nblk + gx - 1) / gx)), dim3(256), 0, ctx->stream, in,
+                     nrow, ctx->n[0], nq, wrap, out);
 }
 
 // gradient of a layer's weights into out and of its biases into db; the
