@@ -305,8 +305,11 @@ inline std::tuple<int, int, int, int, int, int, int, int, int, int> shape_key(co
 // the derived shape on.  time(shape, ms) gives 0, or an error code that ends
 // the search, or a negative value where the shape does not fit;
 // rows_ready() makes the row tiles of the second projection form and says
-// whether there are any.  No shape is timed twice.  best and tbest receive
-// the fastest shape and its time.
+// whether there are any.  best and tbest receive the fastest shape and its
+// time.  No shape is timed twice but the derived one: its first timing may
+// run at the clocks of an idle GPU (72^3, 160 bands FP64 in a new process:
+// one row a thread, 682 us a call, was kept over the derived 596), so it is
+// timed again after the first candidates.
 //
 // Each field's whole range is timed, also where the derived shape already
 // holds the value that is fastest on large grids: 36^3, 20 bands FP32 run
@@ -347,6 +350,15 @@ int search_shape(const HpsiGrid &gr, size_t s, int nb, Time time, Rows rows_read
       c.zlen = 0;
       consider(c);
     }
+  if (!rc) {
+    float t = 0.f;
+    rc = time(timed.front(), t);
+    if (rc) return rc;
+    if (t < tbest) {
+      tbest = t;
+      best = timed.front();
+    }
+  }
   if (best.rx == 2) {  // neighbouring divisors of n2
     int lo = 0, hi = 0;
     for (int t = best.ty - best.ry; t > 0 && !lo; t -= best.ry)

@@ -3,10 +3,11 @@
 // output line.
 //   resolve n1 n2 n3 md size nb nonlocal analytic nseg  ry ty zlen chunk bt rx psplit max_chunk
 //     -> ry ty zlen chunk bt rx psplit fits
-//   search n1 n2 n3 md size nb nonlocal analytic nseg  ry rx psplit chunk
+//   search n1 n2 n3 md size nb nonlocal analytic nseg  ry rx psplit chunk ty cold
 //     the autotuner's search with a clock that prefers these values (0: no
-//     preference) -> the count of timed shapes, the best shape, and each
-//     shape timed, in order: ry ty zlen chunk bt order rx proj plds psplit
+//     preference; cold: the first timing takes twice as long) -> the count
+//     of timed shapes, the best shape, and each shape timed, in order:
+//     ry ty zlen chunk bt order rx proj plds psplit
 #include <cstdio>
 #include <iostream>
 #include <sstream>
@@ -39,7 +40,8 @@ int search(std::istream &in) {
   int nb = 0;
   const HpsiGrid g = read_grid(in, s, nb);
   HpsiShape want, best;
-  in >> want.ry >> want.rx >> want.psplit >> want.chunk;
+  int cold = 0;
+  in >> want.ry >> want.rx >> want.psplit >> want.chunk >> want.ty >> cold;
   std::vector<HpsiShape> seen;
   float t = 0.f;
   const int rc = search_shape(
@@ -48,8 +50,9 @@ int search(std::istream &in) {
         if (!fits(g, h, s)) return -1;
         seen.push_back(h);
         ms = 100.f;
-        for (auto f : {&HpsiShape::ry, &HpsiShape::rx, &HpsiShape::psplit, &HpsiShape::chunk})
+        for (auto f : {&HpsiShape::ry, &HpsiShape::rx, &HpsiShape::psplit, &HpsiShape::chunk, &HpsiShape::ty})
           if (want.*f && h.*f == want.*f) ms -= 10.f;
+        if (cold && seen.size() == 1) ms *= 2.f;
         return 0;
       },
       [] { return true; }, best, t);
