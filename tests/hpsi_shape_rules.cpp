@@ -5,7 +5,8 @@
 //     -> ry ty zlen chunk bt rx psplit fits
 //   search n1 n2 n3 md size nb nonlocal analytic nseg  ry rx psplit chunk ty cold
 //     the autotuner's search with a clock that prefers these values (0: no
-//     preference; cold: the first timing takes twice as long) -> the count
+//     preference; cold 1: the first timing takes twice as long, 3: every third
+//     half as long) -> the count
 //     of timed shapes, the best shape, and each shape timed, in order:
 //     ry ty zlen chunk bt order rx proj plds psplit
 #include <cstdio>
@@ -52,7 +53,8 @@ int search(std::istream &in) {
         ms = 100.f;
         for (auto f : {&HpsiShape::ry, &HpsiShape::rx, &HpsiShape::psplit, &HpsiShape::chunk, &HpsiShape::ty})
           if (want.*f && h.*f == want.*f) ms -= 10.f;
-        if (cold && seen.size() == 1) ms *= 2.f;
+        if (cold == 1 && seen.size() == 1) ms *= 2.f;
+        if (cold == 3 && seen.size() % 3 == 0) ms *= 0.5f;
         return 0;
       },
       [] { return true; }, best, t);

@@ -155,3 +155,11 @@ def test_a_slow_first_timing_does_not_decide(rules, n, size):
     derived, = rules([_resolve(n, size=size, nb=160)])
     best, timed = _search(rules, n, size, 160, cold=1, **{k: derived[k] for k in ("ry", "rx", "psplit", "chunk", "ty")})
     assert best == timed[0]
+
+
+@pytest.mark.parametrize("n,size", [((72, 72, 72), 8), ((36, 36, 36), 4)])
+def test_timings_that_are_low_once_do_not_move_the_shape(rules, n, size):
+    """Every third timing comes out a little low: a candidate has to win again."""
+    derived, = rules([_resolve(n, size=size, nb=160)])
+    best, timed = _search(rules, n, size, 160, cold=3, **{k: derived[k] for k in ("ry", "rx", "psplit", "chunk", "ty")})
+    assert best == timed[0]
